@@ -26,61 +26,11 @@
 #include "mh_device.hpp"
 #include "mh_host.hpp"
 #include "mh_mfma.hpp"
+#include "mh_q4gemm.hpp"
 
 namespace {
 
-using mh::bf16x2_t;
-using mh::bf16x8_t;
-using mh::dma16;
-using mh::dma16s;
-using mh::dma4;
-using mh::f32x16_t;
-using mh::f32x2_t;
-using mh::glb_ptr;
-using mh::lgkm_wait;
-using mh::tie_regs;
-using mh::lds_ptr;
-using mh::lds_read16;
-using mh::lds_read16_at;
-using mh::lds_read4;
-using mh::lds_read4_at;
-using mh::pack_bf16;
-using mh::wait_vmcnt;
-
-constexpr int kBK = 64;
-
-enum Epi { EPI_STORE = 0, EPI_GATE_UP = 1, EPI_SWIGLU = 2 };
-
-struct GemmArgs {
-    const uint16_t* a;       // [a_rows, k] bf16
-    const uint32_t* gather;  // row i of the tile reads a[gather[i]]; null: a[i]
-    const uint32_t* c0; const uint16_t* s0; const uint16_t* b0;  // gate / the matrix
-    const uint32_t* c1; const uint16_t* s1; const uint16_t* b1;  // up
-    uint16_t* out0;          // [s_rows, n]: C, gate, or act
-    uint16_t* out1;          // [s_rows, n]: up (EPI_GATE_UP)
-    const uint4* blocks;     // block map; null: a dense product (entries computed)
-    uint32_t k, n, s_rows, a_rows, w_rows;
-    uint32_t dense_bm;       // rows per entry of a dense product (k_seg)
-    uint32_t ordered;        // k_seg: the map is in launch order (entry b for workgroup b)
-    uint64_t* stamps;        // per workgroup MH_PREFILL_STAMPS words (stamped k_seg only), or null
-};
-
-// One Q4 word (8 codes, low nibble first) -> bf16(fma(s, q, b)) x 8.  High
-// nibbles are converted as 16q and scaled by s/16: the product is exactly
-// q*s, so every value is the one-rounding fma of the reference dequant.
-__device__ __forceinline__ bf16x8_t deq_word(uint32_t w, float s, float s16, float b) {
-    const uint32_t lo = mh::opaque(w & 0x0f0f0f0fu);
-    const uint32_t hi = mh::opaque(w & 0xf0f0f0f0u);
-    uint32_t p[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const float v0 = __builtin_fmaf(mh::ubyte_f32(lo, j), s, b);
-        const float v1 = __builtin_fmaf(mh::ubyte_f32(hi, j), s16, b);
-        p[j] = pack_bf16(v0, v1);
-    }
-    const uint4 u = make_uint4(p[0], p[1], p[2], p[3]);
-    return __builtin_bit_cast(bf16x8_t, u);
-}
+using namespace mh;
 
 // Workgroup -> block-map entry.  Entries come in groups of nt = n / bn (the
 // column tiles of one expert row tile, which read the same A rows); groups
@@ -258,11 +208,10 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void k_grouped(GemmArgs a
             tie_regs(sw);
             tie_regs(bw);
             const uint32_t half = (kb & 1u) ? 0u : 16u;  // bf16 of group kb in the high half
-            float sf[NB], s16[NB], bf[NB];
+            float sf[NB], bf[NB];
 #pragma unroll
             for (int t = 0; t < NB; ++t) {
                 sf[t] = __uint_as_float((sw[t] << half) & 0xffff0000u);
-                s16[t] = sf[t] * 0.0625f;
                 bf[t] = __uint_as_float((bw[t] << half) & 0xffff0000u);
             }
 #pragma unroll
@@ -271,7 +220,7 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void k_grouped(GemmArgs a
 #pragma unroll
                 for (int t = 0; t < NB; ++t) {
                     const uint32_t wv = j == 0 ? bcode[t].x : j == 1 ? bcode[t].y : j == 2 ? bcode[t].z : bcode[t].w;
-                    bfr[t] = deq_word(wv, sf[t], s16[t], bf[t]);
+                    bfr[t] = deq_word(wv, sf[t], bf[t]);
                 }
                 uint4 av[RB];
 #pragma unroll
@@ -368,33 +317,6 @@ __device__ __forceinline__ void mfma_vacc_ready(f32x16_t& c0, f32x16_t& c1) {
 #define MH_SEG_STAGES 3
 #endif
 constexpr int kSegStages = MH_SEG_STAGES;  // LDS ring depth
-
-// Compile-time loop: f(std::integral_constant<int, i>) for i in [0, N).
-template <int I, int N, typename F>
-__device__ __forceinline__ void static_for_impl(F&& f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for_impl<I + 1, N>(f);
-    }
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-    static_for_impl<0, N>(f);
-}
-
-// Fast SiLU for the GEMM epilogue (the gate/up values it sees already
-// carry MFMA accumulation error): g * 1 / (1 + 2^(-g log2 e)) with the
-// hardware exp2 and reciprocal (1 ulp each).
-__device__ __forceinline__ float silu_hw(float g) {
-    const float e = __builtin_amdgcn_exp2f(g * -1.4426950408889634f);
-    return g * __builtin_amdgcn_rcpf(1.0f + e);
-}
-
-__device__ __forceinline__ float bf16_round_hw(float v) {
-    const f32x2_t p = {v, 0.0f};
-    const uint32_t u = __builtin_bit_cast(uint32_t, __builtin_convertvector(p, bf16x2_t));
-    return __uint_as_float(u << 16);
-}
 
 // Wait until at most c (<= C) later stages of OPS vector memory ops each are
 // still in flight.
@@ -626,13 +548,12 @@ __device__ __forceinline__ void seg_pass(const GemmArgs& a, uint32_t brow, uint3
         const uint32_t ab = lds0 + (kb % 3u) * L::A_STAGE + aoff[j];
         static_for<RB>([&](auto rb) { av[rb] = lds_read16_at<rb * 4096>(ab); });
     };
-    float sf[NB], s16[NB], bf[NB];
+    float sf[NB], bf[NB];
     auto scale_bias = [&](uint32_t kb, const uint32_t (&sbw)[2 * NB]) {
         const uint32_t half = (kb & 1u) ? 0u : 16u;  // group kb's bf16 is the high half when kb is odd
 #pragma unroll
         for (int t = 0; t < NB; ++t) {
             sf[t] = __uint_as_float((sbw[2 * t] << half) & 0xffff0000u);
-            s16[t] = sf[t] * 0.0625f;
             bf[t] = __uint_as_float((sbw[2 * t + 1] << half) & 0xffff0000u);
         }
     };
@@ -654,7 +575,7 @@ __device__ __forceinline__ void seg_pass(const GemmArgs& a, uint32_t brow, uint3
     scale_bias(0, sbw);
 #pragma unroll
     for (int t = 0; t < NB; ++t) {
-        bfr[0][t] = deq_word(bc[t].x, sf[t], s16[t], bf[t]);
+        bfr[0][t] = deq_word(bc[t].x, sf[t], bf[t]);
     }
     __builtin_amdgcn_s_barrier();
     read_a(0, 0, av[0]);
@@ -681,7 +602,7 @@ __device__ __forceinline__ void seg_pass(const GemmArgs& a, uint32_t brow, uint3
 #pragma unroll
                     for (int t = 0; t < NB; ++t) {
                         const uint32_t wv = j == 0 ? bc[t].y : j == 1 ? bc[t].z : bc[t].w;
-                        bfr[nxt][t] = deq_word(wv, sf[t], s16[t], bf[t]);
+                        bfr[nxt][t] = deq_word(wv, sf[t], bf[t]);
                     }
                 }
                 // group kb + 2's loads, one after each row block's MFMAs:
@@ -719,7 +640,7 @@ __device__ __forceinline__ void seg_pass(const GemmArgs& a, uint32_t brow, uint3
                     scale_bias(kb + 1, sbw);
 #pragma unroll
                     for (int t = 0; t < NB; ++t) {
-                        bfr[0][t] = deq_word(bc[t].x, sf[t], s16[t], bf[t]);
+                        bfr[0][t] = deq_word(bc[t].x, sf[t], bf[t]);
                     }
                 }
             }
@@ -740,71 +661,8 @@ __device__ __forceinline__ void seg_pass(const GemmArgs& a, uint32_t brow, uint3
     // every wave is done with the ring before another pass refills it
     __builtin_amdgcn_s_barrier();
 
-    // ---- epilogue.  The MFMAs computed C^T (W fragment as the first
-    // operand): lane (i32, h) holds row mp0 + 32 rb + i32 and, at q = 4p + r,
-    // column 8p + 4h + r of its 32-column block.  Values become bf16 pairs;
-    // permlane32_swap of the (p even, p odd) pairs gives lane h = 0 columns
-    // 8p..8p+7 of p = 0, 2 and lane h = 1 those of p = 1, 3, stored 16 bytes
-    // at a time.
-    const mh::gbytes ob0 = mh::uniform_ptr(reinterpret_cast<const char*>(a.out0));
-    const mh::gbytes ob1 = mh::uniform_ptr(reinterpret_cast<const char*>(a.out1 ? a.out1 : a.out0));
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-        const uint32_t row = mp0 + rb * 32u + static_cast<uint32_t>(i32);
-#pragma unroll
-        for (int cb = 0; cb < NBW; ++cb) {
-            constexpr int NOUT = (EPI == EPI_GATE_UP) ? 2 : 1;
-            uint32_t w[NOUT][4][2];  // [output][p][pair]
-#pragma unroll
-            for (int p = 0; p < 4; ++p) {
-                float v[NOUT][4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int q = 4 * p + r;
-                    if constexpr (EPI == EPI_SWIGLU) {
-                        const float g = bf16_round_hw(acc[0][rb][cb][q]);
-                        const float u = bf16_round_hw(acc[1][rb][cb][q]);
-                        v[0][r] = bf16_round_hw(silu_hw(g)) * u;
-                    } else {
-#pragma unroll
-                        for (int o = 0; o < NOUT; ++o) {
-                            v[o][r] = acc[o][rb][cb][q];
-                        }
-                    }
-                }
-#pragma unroll
-                for (int o = 0; o < NOUT; ++o) {
-                    w[o][p][0] = pack_bf16(v[o][0], v[o][1]);
-                    w[o][p][1] = pack_bf16(v[o][2], v[o][3]);
-                }
-            }
-            const uint32_t col = n0 + static_cast<uint32_t>((wave * NBW + cb) * 32 + 8 * h);
-            const uint32_t off = (row * a.n + col) * 2u;
-#pragma unroll
-            for (int o = 0; o < NOUT; ++o) {
-#pragma unroll
-                for (int pp = 0; pp < 2; ++pp) {
-#pragma unroll
-                    for (int d = 0; d < 2; ++d) {
-                        const auto r = __builtin_amdgcn_permlane32_swap(w[o][2 * pp][d], w[o][2 * pp + 1][d], false, false);
-                        w[o][2 * pp][d] = r[0];
-                        w[o][2 * pp + 1][d] = r[1];
-                    }
-                }
-                if (row < m_end) {
-                    const mh::gbytes ob = o == 0 ? ob0 : ob1;
-                    typedef __attribute__((address_space(1))) mh::u32x4* g4;
-                    // columns 8h .. 8h+7 (pp = 0) and 16 + 8h .. (pp = 1)
-                    *reinterpret_cast<g4>(const_cast<char __attribute__((address_space(1)))*>(ob) + off) =
-                        mh::u32x4{w[o][0][0], w[o][0][1], w[o][1][0], w[o][1][1]};
-                    *reinterpret_cast<g4>(const_cast<char __attribute__((address_space(1)))*>(ob) + off + 32u) =
-                        mh::u32x4{w[o][2][0], w[o][2][1], w[o][3][0], w[o][3][1]};
-                }
-            }
-        }
-    }
+    seg_store<RB, NBW, NMAT, EPI>(a, acc, n0, mp0, m_end, i32, h, wave);
 }
-
 
 // Balanced workgroup -> entry mapping of the segment kernels.  A "group" is
 // nt consecutive map entries (one expert row tile across its column tiles,
