@@ -1,4 +1,5 @@
-// mh_q4gemm.hpp -- what the Q4 matrix-product kernels share: their argument block, the dequantization of a code word
+// mh_q4gemm.hpp -- what the Q4 matrix-product kernels share (grouped_gemm.hip,
+// thin_gemm.hip): their argument block, the dequantization of a code word
 // into an MFMA fragment, and the epilogue that stores a wave's tiles.
 #pragma once
 
@@ -25,6 +26,11 @@ struct GemmArgs {
     uint32_t ordered;        // k_seg: the map is in launch order (entry b for workgroup b)
     uint64_t* stamps;        // per workgroup MH_PREFILL_STAMPS words (stamped k_seg only), or null
 };
+
+// thin_gemm.hip: launch-ordered products with few rows per expert.
+bool thin_fits(const GemmArgs& a, uint32_t n_experts, uint32_t bn);
+int gemm_gu_act_thin(const GemmArgs& a, uint32_t n_entries, uint32_t n_experts, hipStream_t s);
+int gemm_grouped_thin(const GemmArgs& a, uint32_t n_entries, uint32_t n_experts, hipStream_t s);
 
 // One Q4 word (8 codes, low nibble first) -> bf16(fma(s, q, b)) x 8.  A code
 // in a byte of its own is the fp8 (e4m3) denormal q 2^-9, so one scaled

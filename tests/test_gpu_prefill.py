@@ -503,3 +503,50 @@ def test_dense_gemm_segment_path(dev, orc, m, n, k):
     want = orc.gemm_q4_grouped(a, w, blocks, len(ents), n, 64)
     rows = np.r_[0:256, 1024:m]
     assert_close(got[rows], want[rows], f"dense segment path {m}x{n}x{k}")
+
+
+@pytest.mark.parametrize("e,h,inter,m,skewed", [
+    # up to 8 rows per expert in the mean (one row block per pass), and past it
+    (64, 512, 512, 1, False), (64, 512, 512, 33, False), (64, 512, 512, 128, False), (64, 512, 512, 129, False),
+    # an expert with every token: passes of 32 rows, and of 128 with a remainder
+    (64, 512, 512, 128, True), (64, 1536, 512, 300, True),
+    # few workgroups: the last mean that runs here and the first that does not
+    (16, 512, 1024, 128, False), (16, 512, 1024, 132, False),
+    # many: one and two passes of the segments, the last mean that runs here
+    (64, 2048, 1024, 1025, False), (64, 2048, 1024, 2304, False)])
+def test_moe_prefill_few_rows_matches_segment_kernel(dev, e, h, inter, m, skewed):
+    """The few-row GEMMs (moe_prefill where an expert's mean rows are few)
+    against the segment kernel (its stamped form, which always runs it): the
+    k order of every sum is the same, so act, ed and out are equal bit for
+    bit; the segment kernel's own outputs are checked against the oracle."""
+    _log(f"moe prefill few rows e={e} h={h} inter={inter} m={m} skewed={skewed}")
+    rng = np.random.default_rng(1000 + m)
+    topk = 4
+    gate, up, down = moe_weights(rng, e, h, inter)
+    router = to_dev(router_weights(rng, e, h, f32=True))
+    b = rng.normal(0, 0.05, e).astype(np.float32)
+    if skewed:
+        b[5] = 1.0e4
+    bias = to_dev(b)
+    x = to_dev(layout.synth_bf16(rng, (m, h)))
+    dg, kg = dev_quant(gate)
+    du, ku = dev_quant(up)
+    dd, kd = dev_quant(down)
+    total, offs = hip.moe_prefill_workspace(m, e, topk, h, inter)
+    stamps = zeros_dev((2 * hip.PREFILL_STAMP_WGS * hip.PREFILL_STAMPS,), np.uint64)
+    outs, wss = [], []
+    for stamped in (False, True):
+        ws = zeros_dev((total // 4,), np.uint32)
+        out = zeros_dev((m, h), np.uint16)
+        if stamped:
+            hip.moe_prefill_stamped(router, bias, dg, du, dd, e, topk, x, m, out, ws, total, stamps, mode=0)
+        else:
+            hip.moe_prefill(router, bias, dg, du, dd, e, topk, x, m, out, ws, total, mode=0)
+        outs.append(from_dev(out, np.uint16))
+        wss.append(from_dev(ws, np.uint32))
+    s = m * topk
+    for key, n in (("act", s * inter), ("ed", s * h)):
+        o = offs[key] // 4
+        np.testing.assert_array_equal(wss[0][o:o + n // 2], wss[1][o:o + n // 2], err_msg=key)
+    assert outs[0].any()
+    np.testing.assert_array_equal(outs[0], outs[1])
