@@ -999,6 +999,10 @@ int mh_gemm_q4_dense(const uint16_t* a, uint32_t m, const mh_quant_weights* w, u
     const uint32_t n = w->out_features;
     GemmArgs g = make_args(a, nullptr, m, w, nullptr, c, nullptr, nullptr, m, n);
     const hipStream_t s = mh::as_stream(stream);
+    int rc = MH_OK;
+    if (gemm_dense_slices(a, m, w, c, s, &rc)) {
+        return rc;
+    }
     // segment entries of 256 x 256 when they fill the chip (>= one per CU),
     // else of 128 x 256 when those do (one 4-row-block pass each), provided
     // the segment kernel's 32-bit offsets hold; else 128 x 256 tiles

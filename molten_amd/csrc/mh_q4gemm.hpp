@@ -32,6 +32,10 @@ bool thin_fits(const GemmArgs& a, uint32_t n_experts, uint32_t bn);
 int gemm_gu_act_thin(const GemmArgs& a, uint32_t n_entries, uint32_t n_experts, hipStream_t s);
 int gemm_grouped_thin(const GemmArgs& a, uint32_t n_entries, uint32_t n_experts, hipStream_t s);
 
+// slice_gemm.hip: the dense product with few output tiles; false where its
+// shape or size is not taken.
+bool gemm_dense_slices(const uint16_t* a, uint32_t m, const mh_quant_weights* w, uint16_t* c, hipStream_t s, int* rc);
+
 // One Q4 word (8 codes, low nibble first) -> bf16(fma(s, q, b)) x 8.  A code
 // in a byte of its own is the fp8 (e4m3) denormal q 2^-9, so one scaled
 // conversion gives two codes as f32 q exactly, whatever s: 19 VALU

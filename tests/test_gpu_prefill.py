@@ -550,3 +550,46 @@ def test_moe_prefill_few_rows_matches_segment_kernel(dev, e, h, inter, m, skewed
         np.testing.assert_array_equal(wss[0][o:o + n // 2], wss[1][o:o + n // 2], err_msg=key)
     assert outs[0].any()
     np.testing.assert_array_equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("m,n,k", [
+    # K cut into slices: one row, empty slices (k 128: one block for 8 waves), ragged
+    # rows and blocks, 64-row and 128-row tiles, many columns on few slices
+    (1, 64, 128), (33, 576, 384), (32, 11776, 256), (21, 512, 11776), (300, 2048, 640), (500, 2048, 512), (60, 9216, 256)])
+def test_dense_gemm_small_and_wide_tiles(dev, orc, m, n, k):
+    """Every tile of the dense product: one-hot rows reproduce the dequantized
+    columns exactly, and the first rows, a middle run and the last (partial)
+    tile match the oracle within the GEMM tolerance."""
+    _log(f"dense {m}x{n}x{k}")
+    rng = np.random.default_rng(m + n + k)
+    w = layout.synth_quant(rng, n, k, 4)
+    wd, keep = dev_quant(w)
+    cols = rng.integers(0, k, m)
+    a1 = np.zeros((m, k), np.uint16)
+    a1[np.arange(m), cols] = layout.f32_to_bf16(np.float32(1.0))
+    c = zeros_dev((m + 1, n), np.uint16)
+    hip.gemm_q4_dense(to_dev(a1), m, wd, c)
+    got = from_dev(c, np.uint16)
+    np.testing.assert_array_equal(got[:m], orc.dequant_bf16(w)[:, cols].T)
+    assert not got[m].any()  # nothing past the last row
+    a = layout.synth_bf16(rng, (m, k))
+    hip.gemm_q4_dense(to_dev(a), m, wd, c)
+    rows = np.unique(np.r_[0:min(m, 40), m // 2:min(m, m // 2 + 40), max(0, m - 70):m])
+    blocks, nb = _dense_map(len(rows), n)
+    want = orc.gemm_q4_grouped(np.ascontiguousarray(a[rows]), w, blocks, nb, n, 64)
+    assert_close(from_dev(c, np.uint16)[rows], want, f"dense {m}x{n}x{k}")
+
+
+def test_dense_gemm_unaligned_output(dev, orc):
+    """An output 4-byte but not 8-byte aligned keeps the 128-row tiles."""
+    m, n, k = 40, 128, 512
+    rng = np.random.default_rng(6)
+    w = layout.synth_quant(rng, n, k, 4)
+    wd, keep = dev_quant(w)
+    a = layout.synth_bf16(rng, (m, k))
+    c = zeros_dev((m * n + 2,), np.uint16)
+    hip.gemm_q4_dense(to_dev(a), m, wd, c.data_ptr() + 4)
+    blocks, nb = _dense_map(m, n)
+    got = from_dev(c, np.uint16)
+    assert not got[:2].any()
+    assert_close(got[2:].reshape(m, n), orc.gemm_q4_grouped(a, w, blocks, nb, n, 64), "dense unaligned")
