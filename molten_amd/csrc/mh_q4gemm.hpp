@@ -32,6 +32,9 @@ bool thin_fits(const GemmArgs& a, uint32_t n_experts, uint32_t bn);
 int gemm_gu_act_thin(const GemmArgs& a, uint32_t n_entries, uint32_t n_experts, hipStream_t s);
 int gemm_grouped_thin(const GemmArgs& a, uint32_t n_entries, uint32_t n_experts, hipStream_t s);
 
+// thin_gemm.hip: the dense product (n % 128 == 0, k % 512 == 0, the segment
+// kernel's offset and alignment limits).
+int gemm_dense_thin(const GemmArgs& a, hipStream_t s);
 // slice_gemm.hip: the dense product with few output tiles; false where its
 // shape or size is not taken.
 bool gemm_dense_slices(const uint16_t* a, uint32_t m, const mh_quant_weights* w, uint16_t* c, hipStream_t s, int* rc);

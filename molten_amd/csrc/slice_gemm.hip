@@ -8,7 +8,7 @@
 // waves) and a wave's chain is 256 k: 8.5 us, half of it the launch and the
 // first loads.  What bounds it then is A, which every 32 columns read again
 // from the L2 (64 MB here, about 15 TB/s); from a few hundred workgroups on
-// wider tiles are the better ones.
+// thin_gemm.hip's wider tiles are the better ones.
 #include "mh_device.hpp"
 #include "mh_host.hpp"
 #include "mh_q4gemm.hpp"
@@ -207,7 +207,7 @@ namespace mh {
 // and columns 8.7 8.7 8.8 8.8 (the call's own cost) / 21 25 26 33; 255 x 2048
 // 10.3 9.1 8.9 9.7 / 49 31 33 44; 500 x 2048 18.8 13.2 12.1 10.7; 100 x 6144
 // 14.3 12.2 10.4 9.7; 60 x 11776 14.8 13.3 11.4 17.0.  Past that (255 x 6144:
-// 27 19 16 18) wider tiles are better.
+// 27 19 16 18) the 64 x 128 tiles of thin_gemm.hip take 15.
 bool gemm_dense_slices(const uint16_t* a, uint32_t m, const mh_quant_weights* w, uint16_t* c, hipStream_t s, int* rc) {
     const uint32_t n = w->out_features, k = w->in_features;
     // 128-k blocks, 32-bit byte offsets, 8-byte stores and whole code pieces

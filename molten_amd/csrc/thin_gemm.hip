@@ -1,5 +1,6 @@
-// thin_gemm.hip -- the grouped Q4 GEMMs of the prefill step when an expert
-// has few rows (short prompts, and up to a mean of 144 rows per expert).
+// thin_gemm.hip -- Q4 products on two or three workgroups per CU: the grouped
+// GEMMs of the prefill step when an expert has few rows (short prompts, and up
+// to a mean of 144 rows per expert), and the dense prefill projections.
 //
 // Same products as grouped_gemm.hip's segment kernel over the same
 // launch-ordered maps, bit for bit: the MFMAs of an output run over k in the
@@ -17,7 +18,9 @@
 // Gate/up and down of 64 experts (2048 x 1536, top-4): 100 tokens 55 + 30 us
 // (4.1 TB/s; the segment kernel 94 + 50); the step of 255 tokens 183 -> 136
 // us, of 1023 209 -> 186.  With dequant and MFMAs taken out the loads alone
-// take 50 + 26 us.
+// take 50 + 26 us.  The dense product has no such limit, yet two waves per
+// SIMD also beat the segment kernel's one with its 256-row tiles: 4095 x 6144
+// x 2048 118 -> 100 us (1030 TFLOP/s), 1023 x 6144 x 2048 60 -> 35.
 #include "mh_device.hpp"
 #include "mh_host.hpp"
 #include "mh_q4gemm.hpp"
@@ -27,7 +30,7 @@ namespace {
 using namespace mh;
 
 constexpr int kThinWaves = 4;
-constexpr int kThinJ = 4;  // K <= 512 kThinJ: scales and biases held in registers
+constexpr int kThinJ = 4;  // scale blocks of 512 k held in registers
 
 // dma16s (mh_mfma.hpp) to LDS address lds_base + OFF, M0
 // written and not restored: nothing else in these kernels uses M0 (every load
@@ -122,18 +125,22 @@ __device__ __forceinline__ void thin_pass(const GemmArgs& a, uint32_t brow, uint
             sboff[t] = min(col0 + static_cast<uint32_t>(i32), a.w_rows - 1u) * groups * 2u;
         }
     }
-    // the column's scales (lanes 0-31) and biases (lanes 32-63) of every group,
-    // 512 k an element
+    // the column's scales (lanes 0-31) and biases (lanes 32-63), 512 k an
+    // element: kThinJ scale blocks from block j on
     uint4 sbr[NB][kThinJ];
+    auto load_sb = [&](uint32_t j) {
 #pragma unroll
-    for (int t = 0; t < NB; ++t) {
-        const gbytes src = (h ? bbase[t / NBW] : sbase[t / NBW]) + sboff[t];
+        for (int t = 0; t < NB; ++t) {
+            const gbytes src = (h ? bbase[t / NBW] : sbase[t / NBW]) + sboff[t];
 #pragma unroll
-        for (int j = 0; j < kThinJ; ++j) {
-            const u32x4 v = *reinterpret_cast<const __attribute__((address_space(1))) u32x4*>(src + min(static_cast<uint32_t>(j), nj - 1u) * 16u);
-            sbr[t][j] = make_uint4(v.x, v.y, v.z, v.w);
+            for (int i = 0; i < kThinJ; ++i) {
+                const u32x4 v = *reinterpret_cast<const __attribute__((address_space(1))) u32x4*>(
+                    src + min(j + i, nj - 1u) * 16u);
+                sbr[t][i] = make_uint4(v.x, v.y, v.z, v.w);
+            }
         }
-    }
+    };
+    load_sb(0);
     auto issue_a = [&](uint32_t s) {
         const uint32_t buf = __builtin_amdgcn_readfirstlane(lds0 + (s % NSA) * L::A_SLOT + wave * QA * 1024u);
         const gbytes ag = uniform_ptr(abase + s * 128u);
@@ -278,10 +285,14 @@ __device__ __forceinline__ void thin_pass(const GemmArgs& a, uint32_t brow, uint
         if constexpr (NEXT) {
             lgkm_wait<RB>(bc);
             if constexpr (u == 7) {
+                if ((j + 1u) % kThinJ == 0u) {
+                    load_sb(j + 1u);
+                } else {
 #pragma unroll
-                for (int t = 0; t < NB; ++t)
+                    for (int t = 0; t < NB; ++t)
 #pragma unroll
-                    for (int i = 0; i + 1 < kThinJ; ++i) sbr[t][i] = sbr[t][i + 1];
+                        for (int i = 0; i + 1 < kThinJ; ++i) sbr[t][i] = sbr[t][i + 1];
+                }
             }
             scale_bias((u + 1) & 7);
 #pragma unroll
@@ -307,7 +318,14 @@ __global__ __launch_bounds__(kThinWaves * 64, (ThinLayout<RBMAX, NMAT * NBW>::WG
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t lds0 = static_cast<uint32_t>((uintptr_t)((lds_ptr)lds));
-    const uint4 blk = a.blocks[blockIdx.x];
+    uint4 blk;
+    if (a.blocks == nullptr) {  // dense: row tiles of dense_bm, fastest, by column tiles
+        const uint32_t rt = (a.s_rows + a.dense_bm - 1u) / a.dense_bm;
+        const uint32_t mr = (blockIdx.x % rt) * a.dense_bm, nc = (blockIdx.x / rt) * (kThinWaves * NBW * 32u);
+        blk = make_uint4(mr, nc, nc, min(mr + a.dense_bm, a.s_rows));
+    } else {
+        blk = a.blocks[blockIdx.x];
+    }
     const uint32_t m0 = blk.x, m_end = blk.w;
     if (m0 >= m_end) {
         return;
@@ -340,6 +358,13 @@ int launch_thin(const GemmArgs& a, uint32_t n_entries, hipStream_t s) {
     return launch_status("k_thin");
 }
 
+template <int RBMAX, int NBW>
+int launch_dense(GemmArgs g, hipStream_t s) {
+    g.dense_bm = 32u * RBMAX;
+    const uint32_t tiles = (g.s_rows + g.dense_bm - 1u) / g.dense_bm * (g.n / (kThinWaves * NBW * 32u));
+    return launch_thin<RBMAX, NBW, 1, false, EPI_STORE>(g, tiles, s);
+}
+
 }  // namespace
 
 namespace mh {
@@ -354,7 +379,10 @@ namespace mh {
 // (16 experts of 1024 x 1536, 192 workgroups: mean 32 70 us against 78, mean
 // 100 105 against 94).
 bool thin_fits(const GemmArgs& a, uint32_t n_experts, uint32_t bn) {
-    if (!a.ordered || a.stamps != nullptr || a.k > 512u * kThinJ) {
+    // (scales and biases are read 16 bytes at a time; make_args leaves the
+    // second matrix's null where there is one)
+    if (!a.ordered || a.stamps != nullptr || !aligned(a.s0, 16) || !aligned(a.b0, 16) || !aligned(a.s1, 16) ||
+        !aligned(a.b1, 16)) {
         return false;
     }
     const bool full = n_experts * (a.n / bn) >= 512u;
@@ -373,6 +401,22 @@ int gemm_gu_act_thin(const GemmArgs& a, uint32_t n_entries, uint32_t n_experts, 
 int gemm_grouped_thin(const GemmArgs& a, uint32_t n_entries, uint32_t n_experts, hipStream_t s) {
     return a.s_rows <= 8u * n_experts ? launch_thin<1, 2, 1, false, EPI_STORE>(a, n_entries, s)
                                       : launch_thin<4, 2, 1, false, EPI_STORE>(a, n_entries, s);
+}
+
+// The dense product: the smallest tile that keeps one workgroup per CU, then
+// the widest (rows x columns of 64 x 128, 128 x 128, 128 x 256; us at K
+// 2048): 255 x 6144 15.3 17.5 29.3; 1023 x 2048 16.0 17.8 29.4; 1023 x 6144
+// 36.6 35.1 35.6; 2047 x 6144 64.6 56.4 60.3; 4095 x 6144 122 106.6 99.8;
+// 4095 x 11776 230 203 185.
+int gemm_dense_thin(const GemmArgs& a, hipStream_t s) {
+    auto tiles = [&](uint32_t rows) { return (a.s_rows + rows - 1u) / rows * static_cast<uint64_t>(a.n / 128u); };
+    if (tiles(64u) <= 256u) {
+        return launch_dense<2, 1>(a, s);
+    }
+    if (tiles(128u) <= 768u || a.n % 256u != 0u) {
+        return launch_dense<4, 1>(a, s);
+    }
+    return launch_dense<4, 2>(a, s);
 }
 
 }  // namespace mh

@@ -555,7 +555,9 @@ def test_moe_prefill_few_rows_matches_segment_kernel(dev, e, h, inter, m, skewed
 @pytest.mark.parametrize("m,n,k", [
     # K cut into slices: one row, empty slices (k 128: one block for 8 waves), ragged
     # rows and blocks, 64-row and 128-row tiles, many columns on few slices
-    (1, 64, 128), (33, 576, 384), (32, 11776, 256), (21, 512, 11776), (300, 2048, 640), (500, 2048, 512), (60, 9216, 256)])
+    (1, 64, 128), (33, 576, 384), (32, 11776, 256), (21, 512, 11776), (300, 2048, 640), (500, 2048, 512), (60, 9216, 256),
+    # column tiles of 128 and 256, one workgroup per CU up to many, scales past 2048 k
+    (257, 6144, 512), (700, 2048, 4608), (4100, 2048, 512), (4100, 6144, 512)])
 def test_dense_gemm_small_and_wide_tiles(dev, orc, m, n, k):
     """Every tile of the dense product: one-hot rows reproduce the dequantized
     columns exactly, and the first rows, a middle run and the last (partial)
@@ -578,6 +580,20 @@ def test_dense_gemm_small_and_wide_tiles(dev, orc, m, n, k):
     blocks, nb = _dense_map(len(rows), n)
     want = orc.gemm_q4_grouped(np.ascontiguousarray(a[rows]), w, blocks, nb, n, 64)
     assert_close(from_dev(c, np.uint16)[rows], want, f"dense {m}x{n}x{k}")
+
+
+def test_dense_gemm_segment_kernel_long_sums(dev, orc):
+    """K past 2048 with a 256 x 256 entry per CU: the segment kernel."""
+    m, n, k = 8100, 2048, 2560
+    rng = np.random.default_rng(5)
+    w = layout.synth_quant(rng, n, k, 4)
+    wd, keep = dev_quant(w)
+    cols = rng.integers(0, k, m)
+    a1 = np.zeros((m, k), np.uint16)
+    a1[np.arange(m), cols] = layout.f32_to_bf16(np.float32(1.0))
+    c = zeros_dev((m, n), np.uint16)
+    hip.gemm_q4_dense(to_dev(a1), m, wd, c)
+    np.testing.assert_array_equal(from_dev(c, np.uint16), orc.dequant_bf16(w)[:, cols].T)
 
 
 def test_dense_gemm_unaligned_output(dev, orc):
