@@ -553,7 +553,8 @@ int mh_moe_prefill(const void* router, int router_dtype, const float* bias, int 
                    size_t workspace_bytes, mh_stream_t stream);
 
 /* Measurement only (no reference counterpart): mh_moe_prefill with the two
- * grouped GEMMs stamped per workgroup.  `stamps` holds 2 x
+ * grouped GEMMs on the segment kernel, stamped per workgroup (mh_moe_prefill
+ * itself runs tiles of 128 rows; same bits).  `stamps` holds 2 x
  * MH_PREFILL_STAMP_WGS x MH_PREFILL_STAMPS u64 words (gate/up + SwiGLU, then
  * down); workgroup g of a GEMM writes at g * MH_PREFILL_STAMPS: the 100 MHz
  * constant clock at its start (word 0) and at its end (after its last stores

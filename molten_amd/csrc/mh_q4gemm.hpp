@@ -22,16 +22,17 @@ struct GemmArgs {
     uint16_t* out1;          // [s_rows, n]: up (EPI_GATE_UP)
     const uint4* blocks;     // block map; null: a dense product (entries computed)
     uint32_t k, n, s_rows, a_rows, w_rows;
-    uint32_t dense_bm;       // rows per entry of a dense product (k_seg)
+    uint32_t dense_bm;       // rows per entry of a dense product
+    uint32_t parts;          // k_thin: workgroups per map entry (its passes dealt out in turn)
+    uint32_t part_units;     // k_thin: map rows whose parts are launched part by part
     uint32_t ordered;        // k_seg: the map is in launch order (entry b for workgroup b)
     uint64_t* stamps;        // per workgroup MH_PREFILL_STAMPS words (stamped k_seg only), or null
 };
 
-// thin_gemm.hip: launch-ordered products with few rows per expert.
-bool thin_fits(const GemmArgs& a, uint32_t n_experts, uint32_t bn);
-int gemm_gu_act_thin(const GemmArgs& a, uint32_t n_entries, uint32_t n_experts, hipStream_t s);
-int gemm_grouped_thin(const GemmArgs& a, uint32_t n_entries, uint32_t n_experts, hipStream_t s);
-
+// thin_gemm.hip: launch-ordered products.
+bool thin_fits(const GemmArgs& a, uint32_t bn);
+int gemm_gu_act_thin(const GemmArgs& a, uint32_t n_entries, hipStream_t s);
+int gemm_grouped_thin(const GemmArgs& a, uint32_t n_entries, hipStream_t s);
 // thin_gemm.hip: the dense product (n % 128 == 0, k % 512 == 0, the segment
 // kernel's offset and alignment limits).
 int gemm_dense_thin(const GemmArgs& a, hipStream_t s);

@@ -154,8 +154,8 @@ int prefill(const char* op, const void* router, int router_dtype, const float* b
                                    ids_sorted, slotpos, gu_map, l.max_gu, dn_map, l.max_dn, kBM, kGuBN,
                                    kDnBN, n_inter, d_model, stream, mma, gu_ord, dn_ord));
     if (l.ordered || stamps != nullptr) {
-        // the segment kernels: on the launch-ordered maps (each workgroup reads
-        // its entry, no ranking), and / or stamped
+        // on the launch-ordered maps (each workgroup reads its entry, no
+        // ranking; thin_gemm.hip), or the segment kernels stamped
         const hipStream_t hs = mh::as_stream(stream);
         MH_TRY(mh::gemm_gu_act_seg(x, ids_sorted, m, gate, up, act, l.ordered ? gu_ord : gu_map,
                                    l.ordered ? l.grid_gu : l.max_gu, s, n_inter, kBM, kGuBN, l.ordered, stamps, hs));

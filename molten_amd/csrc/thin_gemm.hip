@@ -1,26 +1,25 @@
 // thin_gemm.hip -- Q4 products on two or three workgroups per CU: the grouped
-// GEMMs of the prefill step when an expert has few rows (short prompts, and up
-// to a mean of 144 rows per expert), and the dense prefill projections.
+// GEMMs of the prefill step (over launch-ordered maps) and the dense prefill
+// projections.
 //
-// Same products as grouped_gemm.hip's segment kernel over the same
-// launch-ordered maps, bit for bit: the MFMAs of an output run over k in the
-// same order.  What differs is what bounds them: reading every chosen
-// expert's weights (5.3 MB each) and turning their codes into bf16 (19 VALU
-// instructions per 8 codes), with the matrix cores mostly idle.  A lone wave
-// issues a VALU instruction every ~5 cycles where a SIMD takes one every 2 to
-// 4, so the tile gives up rows for waves: at most 80 KB of LDS and 256
-// registers, two workgroups per CU (three with one row block), whose loads
-// and dequant cover each other.  A column's scales and biases are read once,
-// whole, into registers (16 bytes at a time from rows of 64, as the segment
-// kernel's LDS blocks take them, each line was fetched up to four times: 310
-// MB instead of 235 for gate/up of 64 experts).
+// Same products as grouped_gemm.hip's segment kernel, bit for bit: the MFMAs
+// of an output run over k in the same order.  With few rows per expert they
+// are bound by reading every chosen expert's weights (5.3 MB each) and turning
+// their codes into bf16 (19 VALU instructions per 8 codes), with many by the
+// matrix cores.  A lone wave issues a VALU instruction every ~5 cycles where a
+// SIMD takes one every 2 to 4, so the tile gives up rows for waves: at most
+// four row blocks of 32 per pass in 80 KB of LDS and 256 registers, two
+// workgroups per CU (three with one row block), whose loads, dequant and
+// MFMAs cover each other.  That pays for dequantizing an expert's codes once
+// per 128 rows instead of once per 288.  A column's scales and biases are read
+// once, whole, into registers (16 bytes at a time from rows of 64, as the
+// segment kernel's LDS blocks take them, each line was fetched up to four
+// times: 310 MB instead of 235 for gate/up of 64 experts).
 //
-// Gate/up and down of 64 experts (2048 x 1536, top-4): 100 tokens 55 + 30 us
-// (4.1 TB/s; the segment kernel 94 + 50); the step of 255 tokens 183 -> 136
-// us, of 1023 209 -> 186.  With dequant and MFMAs taken out the loads alone
-// take 50 + 26 us.  The dense product has no such limit, yet two waves per
-// SIMD also beat the segment kernel's one with its 256-row tiles: 4095 x 6144
-// x 2048 118 -> 100 us (1030 TFLOP/s), 1023 x 6144 x 2048 60 -> 35.
+// Gate/up and down of 64 experts (2048 x 1536, top-4), 100 tokens: 55 + 30 us
+// (4.1 TB/s; the segment kernel 94 + 50); with dequant and MFMAs taken out the
+// loads alone take 50 + 26.  Dense 4095 x 6144 x 2048: 100 us (1030 TFLOP/s;
+// the segment kernel 118), 1023 x 6144 x 2048 35 (60).
 #include "mh_device.hpp"
 #include "mh_host.hpp"
 #include "mh_q4gemm.hpp"
@@ -258,11 +257,13 @@ __device__ __forceinline__ void thin_pass(const GemmArgs& a, uint32_t brow, uint
             const int cur = t & 1, nxt = cur ^ 1;
             read_a(s, t + 1, av[nxt]);
             lgkm_wait<RB>(av[cur]);
-            mma(cur);
+            // (written ahead of this step's MFMAs it is spread over more of them:
+            // 4095 x 11776 x 2048 181 -> 177 us)
 #pragma unroll
             for (int f = 0; f < NB; ++f) {
                 bfr[nxt][f] = deq_word(word(bc[f], t + 1), sf[f], bf[f]);
             }
+            mma(cur);
         }
         // Before the last step: the wave's reads of this A slot are done and
         // its loads of stage s + 1 have landed; the barrier publishes stage
@@ -310,8 +311,13 @@ __device__ __forceinline__ void thin_pass(const GemmArgs& a, uint32_t brow, uint
     seg_store<RB, NBW, NMAT, EPI>(a, acc, n0, mp0, m_end, i32, h, wave);
 }
 
-// One workgroup per entry of a launch-ordered map; an entry's rows in
-// balanced passes of at most RBMAX row blocks.
+// An entry of a launch-ordered map (up to 512 rows of one expert) is covered
+// in balanced passes of at most RBMAX row blocks, dealt out to `parts`
+// workgroups: pass p to workgroup p % parts.  All of an entry's passes read
+// the same codes, so its workgroups run on one XCD and near each other; but
+// parts without a pass end at once, and runs of them as short as an entry's
+// column tiles would leave the live ones on the same few CUs (workgroups are
+// dealt to an XCD's CUs in turn), hence the groups of 16 or more.
 template <int RBMAX, int NBW, int NMAT, bool GATHER, int EPI>
 __global__ __launch_bounds__(kThinWaves * 64, (ThinLayout<RBMAX, NMAT * NBW>::WGS)) void k_thin(GemmArgs a) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
@@ -319,12 +325,21 @@ __global__ __launch_bounds__(kThinWaves * 64, (ThinLayout<RBMAX, NMAT * NBW>::WG
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t lds0 = static_cast<uint32_t>((uintptr_t)((lds_ptr)lds));
     uint4 blk;
+    uint32_t part = 0u, parts = 1u;
     if (a.blocks == nullptr) {  // dense: row tiles of dense_bm, fastest, by column tiles
         const uint32_t rt = (a.s_rows + a.dense_bm - 1u) / a.dense_bm;
         const uint32_t mr = (blockIdx.x % rt) * a.dense_bm, nc = (blockIdx.x / rt) * (kThinWaves * NBW * 32u);
         blk = make_uint4(mr, nc, nc, min(mr + a.dense_bm, a.s_rows));
     } else {
-        blk = a.blocks[blockIdx.x];
+        // groups of part_units map rows (their nt column tiles each): part 0
+        // of the group's entries, then part 1, ...
+        parts = a.parts;
+        const uint32_t nt = a.n / (kThinWaves * NBW * 32u), j = blockIdx.x / 8u;
+        const uint32_t units = gridDim.x / (8u * parts * nt), per = a.part_units * nt;
+        const uint32_t g = j / (per * parts), r = j % (per * parts);
+        const uint32_t size = min(a.part_units, units - g * a.part_units) * nt;
+        part = r / size;
+        blk = a.blocks[(g * per + r % size) * 8u + blockIdx.x % 8u];
     }
     const uint32_t m0 = blk.x, m_end = blk.w;
     if (m0 >= m_end) {
@@ -332,16 +347,15 @@ __global__ __launch_bounds__(kThinWaves * 64, (ThinLayout<RBMAX, NMAT * NBW>::WG
     }
     const uint32_t nrb = (m_end - m0 + 31u) / 32u;
     const uint32_t passes = (nrb + RBMAX - 1u) / RBMAX;
-    uint32_t mp0 = m0;
-    for (uint32_t p = 0; p < passes; ++p) {
-        const uint32_t left = (m_end - mp0 + 31u) / 32u;
-        const uint32_t rb = (left + (passes - p) - 1u) / (passes - p);
+    const uint32_t each = nrb / passes, extra = nrb % passes;
+    for (uint32_t p = part; p < passes; p += parts) {
+        const uint32_t mp0 = m0 + 32u * (p * each + min(p, extra));
+        const uint32_t rb = each + (p < extra ? 1u : 0u);
         static_for<RBMAX>([&](auto i) {
             if (rb == i + 1u) {
                 thin_pass<i + 1, RBMAX, NBW, NMAT, GATHER, EPI>(a, blk.y, blk.z, mp0, m_end, lds0, lane, wave);
             }
         });
-        mp0 += rb * 32u;
     }
 }
 
@@ -354,7 +368,7 @@ int launch_thin(const GemmArgs& a, uint32_t n_entries, hipStream_t s) {
     if (e != hipSuccess) {
         return hip_error(e, "k_thin");
     }
-    hipLaunchKernelGGL(kern, dim3(n_entries), dim3(kThinWaves * 64), lds, s, a);
+    hipLaunchKernelGGL(kern, dim3(a.blocks == nullptr ? n_entries : n_entries * a.parts), dim3(kThinWaves * 64), lds, s, a);
     return launch_status("k_thin");
 }
 
@@ -369,38 +383,45 @@ int launch_dense(GemmArgs g, hipStream_t s) {
 
 namespace mh {
 
-// Rows per expert (the mean; the host does not know the routing) up to which
-// these kernels run the launch-ordered products.  An expert of up to 128 rows
-// is one pass; past that the codes are dequantized once more per pass, and the
-// segment kernel's single pass of 288 rows wins from a mean of about 150
-// (64 experts top-4, step of 2300 tokens: 291 us against 301; 2600: 321
-// against 317).  With fewer workgroups than two per CU the second wave of a
-// SIMD is missing and the segment kernel's deeper row blocking wins earlier
-// (16 experts of 1024 x 1536, 192 workgroups: mean 32 70 us against 78, mean
-// 100 105 against 94).
-bool thin_fits(const GemmArgs& a, uint32_t n_experts, uint32_t bn) {
-    // (scales and biases are read 16 bytes at a time; make_args leaves the
-    // second matrix's null where there is one)
-    if (!a.ordered || a.stamps != nullptr || !aligned(a.s0, 16) || !aligned(a.b0, 16) || !aligned(a.s1, 16) ||
-        !aligned(a.b1, 16)) {
-        return false;
+// Whether these kernels run a launch-ordered product (its offset and
+// alignment limits checked as the segment kernel's).  Scales and biases are
+// read 16 bytes at a time (make_args leaves the second matrix's null where
+// there is one).  Where every expert has 208 to 288 rows the segment kernel
+// covers each in one pass, and with two workgroups' worth of entries per CU
+// it is level or a little better (64 experts, step of 3500, 3800, 4096 tokens
+// routed evenly: 324 344 373 us against 325 347 378; 3000: 295 against 293;
+// routed unevenly, 4096: 405 against 384).  The host knows only the mean.
+bool thin_fits(const GemmArgs& a, uint32_t bn) {
+    const uint32_t n_experts = a.w_rows / a.n;
+    const bool one_pass = n_experts * (a.n / bn) >= 512u && a.s_rows > 208u * n_experts && a.s_rows <= 288u * n_experts;
+    return a.ordered && a.stamps == nullptr && !one_pass && aligned(a.s0, 16) && aligned(a.b0, 16) &&
+           aligned(a.s1, 16) && aligned(a.b1, 16);
+}
+
+template <int NBW, int NMAT, bool GATHER, int EPI>
+static int launch_grouped(GemmArgs g, uint32_t n_entries, uint32_t n_experts, hipStream_t s) {
+    // One row block per pass needs less LDS (three workgroups per CU), but an
+    // expert of more than 32 rows takes several passes then: up to a mean of 4
+    // rows (64 experts top-4: 60 tokens 135.6 us against 138.1).
+    const uint32_t nt = g.n / (kThinWaves * NBW * 32u);
+    g.part_units = (16u + nt - 1u) / nt;
+    if (g.s_rows <= 4u * n_experts) {
+        g.parts = 1u;
+        return launch_thin<1, NBW, NMAT, GATHER, EPI>(g, n_entries, s);
     }
-    const bool full = n_experts * (a.n / bn) >= 512u;
-    return a.s_rows <= (full ? 144u : 32u) * n_experts;
+    // a workgroup for every pass of a 512-row entry (step of 255, 1023, 2048,
+    // 4096 tokens: 133 178 242 392 us; one workgroup per entry 135 187 266
+    // 422, the segment kernel 185 213 285 408)
+    g.parts = 4u;
+    return launch_thin<4, NBW, NMAT, GATHER, EPI>(g, n_entries, s);
 }
 
-// One row block per pass needs a third less LDS (three workgroups per CU)
-// but an expert of more than 32 rows then takes several passes: up to a mean
-// of 8 rows (128 tokens: step 130.9 us against 133.7; 255 tokens, mean 16:
-// 149 against 136).
-int gemm_gu_act_thin(const GemmArgs& a, uint32_t n_entries, uint32_t n_experts, hipStream_t s) {
-    return a.s_rows <= 8u * n_experts ? launch_thin<1, 1, 2, true, EPI_SWIGLU>(a, n_entries, s)
-                                      : launch_thin<4, 1, 2, true, EPI_SWIGLU>(a, n_entries, s);
+int gemm_gu_act_thin(const GemmArgs& a, uint32_t n_entries, hipStream_t s) {
+    return launch_grouped<1, 2, true, EPI_SWIGLU>(a, n_entries, a.w_rows / a.n, s);
 }
 
-int gemm_grouped_thin(const GemmArgs& a, uint32_t n_entries, uint32_t n_experts, hipStream_t s) {
-    return a.s_rows <= 8u * n_experts ? launch_thin<1, 2, 1, false, EPI_STORE>(a, n_entries, s)
-                                      : launch_thin<4, 2, 1, false, EPI_STORE>(a, n_entries, s);
+int gemm_grouped_thin(const GemmArgs& a, uint32_t n_entries, hipStream_t s) {
+    return launch_grouped<2, 1, false, EPI_STORE>(a, n_entries, a.w_rows / a.n, s);
 }
 
 // The dense product: the smallest tile that keeps one workgroup per CU, then

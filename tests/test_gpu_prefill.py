@@ -506,20 +506,19 @@ def test_dense_gemm_segment_path(dev, orc, m, n, k):
 
 
 @pytest.mark.parametrize("e,h,inter,m,skewed", [
-    # up to 8 rows per expert in the mean (one row block per pass), and past it
-    (64, 512, 512, 1, False), (64, 512, 512, 33, False), (64, 512, 512, 128, False), (64, 512, 512, 129, False),
-    # an expert with every token: passes of 32 rows, and of 128 with a remainder
-    (64, 512, 512, 128, True), (64, 1536, 512, 300, True),
-    # few workgroups: the last mean that runs here and the first that does not
-    (16, 512, 1024, 128, False), (16, 512, 1024, 132, False),
-    # many: one and two passes of the segments, the last mean that runs here
-    (64, 2048, 1024, 1025, False), (64, 2048, 1024, 2304, False)])
-def test_moe_prefill_few_rows_matches_segment_kernel(dev, e, h, inter, m, skewed):
-    """The few-row GEMMs (moe_prefill where an expert's mean rows are few)
-    against the segment kernel (its stamped form, which always runs it): the
+    # up to 4 rows per expert in the mean (one row block per pass), and past it
+    (64, 512, 512, 1, False), (64, 512, 512, 33, False), (64, 512, 512, 64, False), (64, 512, 512, 65, False),
+    # an expert with every token: two passes of one row block, three and eight of four
+    (64, 512, 512, 60, True), (64, 1536, 512, 300, True), (16, 512, 1024, 1000, True),
+    # column tiles in groups (4, 8, 16 and 24 of them), ragged last passes
+    (16, 1024, 512, 128, False), (64, 2048, 1024, 1025, False), (24, 512, 1536, 700, False),
+    (64, 2048, 1024, 2304, False)])
+def test_moe_prefill_matches_segment_kernel(dev, e, h, inter, m, skewed):
+    """The step's grouped GEMMs against the segment kernel's (the stamped step
+    runs that one): the
     k order of every sum is the same, so act, ed and out are equal bit for
     bit; the segment kernel's own outputs are checked against the oracle."""
-    _log(f"moe prefill few rows e={e} h={h} inter={inter} m={m} skewed={skewed}")
+    _log(f"moe prefill against segments e={e} h={h} inter={inter} m={m} skewed={skewed}")
     rng = np.random.default_rng(1000 + m)
     topk = 4
     gate, up, down = moe_weights(rng, e, h, inter)
