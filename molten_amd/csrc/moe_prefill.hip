@@ -399,8 +399,10 @@ __device__ void write_ordered(uint4* ord, uint32_t rank, uint32_t m0, uint32_t m
 // both block-map offsets by two workgroup scans) and its block's prefix row,
 // scatters block j's slots stably (slot order; ranks within each 64-slot
 // chunk from ballots), writes the block-map entries of experts j, j + G, ...
-// and zeroes its share of both maps' unused tails.  Workgroup 0 writes
-// counts, offsets and the block-map offsets.  With gu_ord / dn_ord, the same
+// and zeroes its share of both maps' unused tails.  With fewer blocks than
+// experts there are workgroups past the blocks for the maps alone (step of 21
+// tokens: two workgroups ranked and wrote every expert's entries, 32 us; one
+// each 8).  Workgroup 0 writes counts, offsets and the block-map offsets.  With gu_ord / dn_ord, the same
 // entries again in launch order (unused workgroups' entries zero).
 __global__ __launch_bounds__(256) void k_scatter_maps(const uint32_t* ids, const uint32_t* pre, const uint32_t* tot,
                                                       uint32_t m, uint32_t e, uint32_t topk, uint32_t* counts,
@@ -409,7 +411,7 @@ __global__ __launch_bounds__(256) void k_scatter_maps(const uint32_t* ids, const
                                                       uint32_t max_gu, uint4* dn, uint32_t max_dn, uint32_t bm,
                                                       uint32_t gu_bn, uint32_t dn_bn, uint32_t gu_n, uint32_t dn_n,
                                                       uint4* gu_ord, uint4* dn_ord, uint32_t gu_grid,
-                                                      uint32_t dn_grid) {
+                                                      uint32_t dn_grid, uint32_t nblk) {
     __shared__ uint32_t tot_l[mh::kMaxExperts], off_l[mh::kMaxExperts], base_l[mh::kMaxExperts],
         rb_l[mh::kMaxExperts];
     __shared__ uint32_t chist[4][mh::kMaxExperts];
@@ -417,10 +419,10 @@ __global__ __launch_bounds__(256) void k_scatter_maps(const uint32_t* ids, const
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t j = blockIdx.x;
     const uint32_t total = tid < e ? tot[tid] : 0u;
-    const uint32_t before = tid < e ? pre[static_cast<size_t>(j) * e + tid] : 0u;
+    const uint32_t before = tid < e && j < nblk ? pre[static_cast<size_t>(j) * e + tid] : 0u;
     // this block's slots (at most 256, one per thread)
     const uint32_t s0 = j * kRouteBlock * topk;
-    const uint32_t ns = min(kRouteBlock, m - j * kRouteBlock) * topk;
+    const uint32_t ns = j < nblk ? min(kRouteBlock, m - j * kRouteBlock) * topk : 0u;
     const bool act = tid < ns;
     const uint32_t v = act ? ids[s0 + tid] : 0xffffffffu;
     uint32_t all;
@@ -653,11 +655,11 @@ int moe_route_sort_maps(const float* logits, const float* bias, int mode, float 
                       max_gu / gu_tiles <= mh::kMaxOrderedRows,
                   MH_ERR_UNSUPPORTED, "prefill routing: launch-ordered maps of %u rows", max_gu / gu_tiles);
     }
-    hipLaunchKernelGGL(k_scatter_maps, dim3(nblk), dim3(256), 0, st, ids, hb, tot, m, e, topk, counts, offsets,
+    hipLaunchKernelGGL(k_scatter_maps, dim3(nblk > e ? nblk : e), dim3(256), 0, st, ids, hb, tot, m, e, topk, counts, offsets,
                        gu_off, dn_off, ids_sorted, slotpos, reinterpret_cast<uint4*>(gu), max_gu,
                        reinterpret_cast<uint4*>(dn), max_dn, bm, gu_bn, dn_bn, gu_n, dn_n,
                        reinterpret_cast<uint4*>(gu_ord), reinterpret_cast<uint4*>(dn_ord),
-                       mh::map_grid(max_gu, gu_tiles), mh::map_grid(max_dn, dn_tiles));
+                       mh::map_grid(max_gu, gu_tiles), mh::map_grid(max_dn, dn_tiles), nblk);
     return mh::launch_status("k_scatter_maps");
 }
 
