@@ -176,7 +176,7 @@ __global__ __launch_bounds__(kThreads) void k_dense_gemv(DenseArgs a) {
 }
 
 // Router logits of many tokens, tiled: a workgroup takes kRtTokens tokens
-// and kRtExperts experts; the experts' rows are staged once in the LDS as
+// and kRtExperts (even) experts; the experts' rows are staged once in the LDS as
 // f32 (chunk c of row e as 8 pieces of 16 bytes, piece q at q ^ ((c >> 1) &
 // 7), so the 16 lanes of a 16-byte read cover all 64 banks once), then each
 // wave runs its tokens in groups of four with x in registers (lane c holds
@@ -191,13 +191,11 @@ __global__ __launch_bounds__(kThreads) void k_dense_gemv(DenseArgs a) {
 // leaving value v in lane 8v + 7; the chunk order's +0 is applied once to
 // that sum (an IEEE sum is -0 only when both operands are, so the bits are
 // the same).  W comes from the L2 once per workgroup.
-constexpr int kRtTokens = 64;
-constexpr int kRtExperts = 8;
-constexpr int kRtGroup = 4;                                // tokens per group
-constexpr int kRtGroups = kRtTokens / (kRtGroup * kWaves);  // groups per wave
+constexpr int kRtGroup = 4;  // tokens per group
 
-template <typename WT>
+template <typename WT, int kRtTokens, int kRtExperts>
 __global__ __launch_bounds__(kThreads, 2) void k_router_tiles(DenseArgs a) {
+    constexpr int kRtGroups = kRtTokens / (kRtGroup * kWaves);  // groups per wave
     extern __shared__ float wl[];  // [kRtExperts][C][8 pieces][4]
     __shared__ float zl[kRtTokens][kRtExperts];
     __shared__ __attribute__((aligned(16))) float tl[kWaves][8 * 64];  // a wave's chain values, [value][chunk]
@@ -327,18 +325,33 @@ __global__ __launch_bounds__(kThreads, 2) void k_router_tiles(DenseArgs a) {
     }
 }
 
-template <typename WT>
-int launch_router_tiles(const DenseArgs& a, hipStream_t stream) {
+template <typename WT, int TOKENS, int EXPERTS>
+int launch_router_tiles_as(const DenseArgs& a, hipStream_t stream) {
     const uint32_t C = a.k / 32u;
-    const size_t lds = static_cast<size_t>(kRtExperts) * C * 32u * sizeof(float);
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_router_tiles<WT>),
+    const size_t lds = static_cast<size_t>(EXPERTS) * C * 32u * sizeof(float);
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_router_tiles<WT, TOKENS, EXPERTS>),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
     if (e != hipSuccess) {
         return mh::hip_error(e, "k_router_tiles: LDS attribute");
     }
-    const dim3 grid((a.m + kRtTokens - 1) / kRtTokens, (a.n + kRtExperts - 1) / kRtExperts);
-    hipLaunchKernelGGL(k_router_tiles<WT>, grid, dim3(kThreads), lds, stream, a);
+    const dim3 grid((a.m + TOKENS - 1) / TOKENS, (a.n + EXPERTS - 1) / EXPERTS);
+    hipLaunchKernelGGL((k_router_tiles<WT, TOKENS, EXPERTS>), grid, dim3(kThreads), lds, stream, a);
     return mh::launch_status("k_router_tiles");
+}
+
+template <typename WT>
+int launch_router_tiles(const DenseArgs& a, hipStream_t stream) {
+    // smaller tiles while they are what fills the chip (a tile of 64 x 8 is a
+    // chain of ~20 us however few there are): f32 router of 64 experts, step
+    // of 21 255 500 1023 2048 4096 tokens by tile, 64 x 8: 115 134 150 179 250
+    // 390 us; 16 x 8: 103 122 139 169 247 406; 16 x 2: 98 117 139 174 257 421
+    if (a.m <= 512u) {
+        return launch_router_tiles_as<WT, 16, 2>(a, stream);
+    }
+    if (a.m <= 2048u) {
+        return launch_router_tiles_as<WT, 16, 8>(a, stream);
+    }
+    return launch_router_tiles_as<WT, 64, 8>(a, stream);
 }
 
 // Decode router logits only (the routing runs in the expert kernel): one
