@@ -213,17 +213,28 @@ def _ptr(t) -> Optional[int]:
     return t.data_ptr()
 
 
+_raw_stream = None  # (torch's raw-stream getter, current-device getter), once torch has a GPU
+
+
 def _stream(stream) -> Optional[int]:
+    """The stream to launch on: the given one, else the calling thread's
+    current torch stream on its current device, asked for at every call.  The
+    raw getter is one C call (0.3 us); torch.cuda.current_stream() behind
+    torch.cuda.is_available() took 3.5 of the 8.3 us of a GEMV call."""
     if stream is not None:
         return stream if isinstance(stream, int) else stream.cuda_stream
+    global _raw_stream
     try:
-        import torch
+        if _raw_stream is None:
+            import torch
 
-        if torch.cuda.is_available():
-            return torch.cuda.current_stream().cuda_stream
+            if not torch.cuda.is_available():
+                return None
+            torch.cuda.init()
+            _raw_stream = (torch._C._cuda_getCurrentRawStream, torch.cuda.current_device)
+        return _raw_stream[0](_raw_stream[1]())
     except Exception:  # pragma: no cover - torch import failure
-        pass
-    return None
+        return None
 
 
 STATUS_ARGMAX_WAIT = 1

@@ -297,3 +297,37 @@ def test_python_mirrors_of_header_constants():
     names = [w.strip().split("=")[0].strip() for w in enum.split(",") if w.strip()]
     assert names[-1] == "MH_PREFILL_WS_REGIONS"
     assert [n[len("MH_PREFILL_WS_"):].lower() for n in names[:-1]] == hip.PREFILL_WS_REGIONS
+
+
+@pytest.mark.gpu
+def test_default_stream_is_the_threads_current_one(dev):
+    """Without a stream argument a call goes to the calling thread's current
+    torch stream: the default one, a side stream inside its context, and each
+    thread's own."""
+    import threading
+
+    import torch
+
+    def seen():
+        return hip._stream(None), torch.cuda.current_stream().cuda_stream
+
+    got, want = seen()
+    assert got == want
+    side, other = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        assert seen() == (side.cuda_stream, side.cuda_stream)
+        inner = []
+
+        def work():
+            with torch.cuda.stream(other):
+                inner.append(seen())
+            inner.append(seen())
+
+        t = threading.Thread(target=work)
+        t.start()
+        t.join()
+        assert inner[0] == (other.cuda_stream, other.cuda_stream)
+        assert inner[1][0] == inner[1][1]
+        assert seen() == (side.cuda_stream, side.cuda_stream)
+    assert seen() == (got, want)
+    assert hip._stream(side) == side.cuda_stream and hip._stream(7) == 7
