@@ -317,7 +317,7 @@ __device__ __forceinline__ void thin_pass(const GemmArgs& a, uint32_t brow, uint
 // the same codes, so its workgroups run on one XCD and near each other; but
 // parts without a pass end at once, and runs of them as short as an entry's
 // column tiles would leave the live ones on the same few CUs (workgroups are
-// dealt to an XCD's CUs in turn), hence the groups of 16 or more.
+// dealt to an XCD's 32 CUs in turn), hence the groups of 32 tiles or more.
 template <int RBMAX, int NBW, int NMAT, bool GATHER, int EPI>
 __global__ __launch_bounds__(kThinWaves * 64, (ThinLayout<RBMAX, NMAT * NBW>::WGS)) void k_thin(GemmArgs a) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
@@ -404,7 +404,7 @@ static int launch_grouped(GemmArgs g, uint32_t n_entries, uint32_t n_experts, hi
     // expert of more than 32 rows takes several passes then: up to a mean of 4
     // rows (64 experts top-4: 60 tokens 135.6 us against 138.1).
     const uint32_t nt = g.n / (kThinWaves * NBW * 32u);
-    g.part_units = (16u + nt - 1u) / nt;
+    g.part_units = (32u + nt - 1u) / nt;
     if (g.s_rows <= 4u * n_experts) {
         g.parts = 1u;
         return launch_thin<1, NBW, NMAT, GATHER, EPI>(g, n_entries, s);
