@@ -213,28 +213,35 @@ def _ptr(t) -> Optional[int]:
     return t.data_ptr()
 
 
-_raw_stream = None  # (torch's raw-stream getter, current-device getter), once torch has a GPU
+_raw_stream = None  # (device -> its current stream's handle, current-device getter), once torch has a GPU
 
 
 def _stream(stream) -> Optional[int]:
     """The stream to launch on: the given one, else the calling thread's
-    current torch stream on its current device, asked for at every call.  The
-    raw getter is one C call (0.3 us); torch.cuda.current_stream() behind
-    torch.cuda.is_available() took 3.5 of the 8.3 us of a GEMV call."""
+    current torch stream on its current device, asked for at every call; the
+    null stream without torch or without a GPU that torch can use.  Torch's
+    raw getter is one C call (0.3 us; torch.cuda.current_stream() behind
+    torch.cuda.is_available() took 3.5 of the 8.3 us of a GEMV call) but no
+    public name: a torch without it is asked through the public one.  An
+    error of either is the caller's: on the null stream instead, the launch
+    would not be ordered with the caller's own work."""
     if stream is not None:
         return stream if isinstance(stream, int) else stream.cuda_stream
     global _raw_stream
-    try:
-        if _raw_stream is None:
+    if _raw_stream is None:
+        try:
             import torch
-
-            if not torch.cuda.is_available():
-                return None
-            torch.cuda.init()
-            _raw_stream = (torch._C._cuda_getCurrentRawStream, torch.cuda.current_device)
-        return _raw_stream[0](_raw_stream[1]())
-    except Exception:  # pragma: no cover - torch import failure
-        return None
+        except Exception:  # torch missing or not loadable
+            return None
+        if not torch.cuda.is_available():
+            return None
+        torch.cuda.init()
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        if raw is None:
+            def raw(device):
+                return torch.cuda.current_stream(device).cuda_stream
+        _raw_stream = (raw, torch.cuda.current_device)
+    return _raw_stream[0](_raw_stream[1]())
 
 
 STATUS_ARGMAX_WAIT = 1

@@ -331,3 +331,43 @@ def test_default_stream_is_the_threads_current_one(dev):
         assert seen() == (side.cuda_stream, side.cuda_stream)
     assert seen() == (got, want)
     assert hip._stream(side) == side.cuda_stream and hip._stream(7) == 7
+
+
+def test_default_stream_without_the_raw_getter(monkeypatch):
+    """A torch without the raw-stream getter is asked through its public
+    current_stream, and an error of the lookup reaches the caller: neither
+    may end on the null stream, which a side stream is not ordered with."""
+    import types
+
+    import torch
+
+    asked = []
+
+    def current_stream(device=None):
+        asked.append(device)
+        return types.SimpleNamespace(cuda_stream=0x1234)
+
+    monkeypatch.setattr(hip, "_raw_stream", None)
+    monkeypatch.setattr(torch.cuda, "is_available", lambda: True)
+    monkeypatch.setattr(torch.cuda, "init", lambda: None)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 3)
+    monkeypatch.setattr(torch.cuda, "current_stream", current_stream)
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    assert hip._stream(None) == 0x1234 and asked == [3]
+
+    def broken():
+        raise RuntimeError("no current device")
+
+    monkeypatch.setattr(hip, "_raw_stream", (lambda d: 0, broken))
+    with pytest.raises(RuntimeError, match="no current device"):
+        hip._stream(None)
+
+
+def test_default_stream_without_a_gpu(monkeypatch):
+    """Without a GPU that torch can use: the null stream, and nothing kept."""
+    import torch
+
+    monkeypatch.setattr(hip, "_raw_stream", None)
+    monkeypatch.setattr(torch.cuda, "is_available", lambda: False)
+    assert hip._stream(None) is None
+    assert hip._raw_stream is None
