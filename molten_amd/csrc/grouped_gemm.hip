@@ -1002,18 +1002,26 @@ int mh_gemm_q4_dense(const uint16_t* a, uint32_t m, const mh_quant_weights* w, u
     if (gemm_dense_slices(a, m, w, c, s, &rc)) {
         return rc;
     }
+    const uint32_t segs = (m + 255u) / 256u * (n / 256u), segs128 = (m + 127u) / 128u * (n / 256u);
     if (n % 128 == 0 && w->in_features % 512u == 0 && static_cast<uint64_t>(m) * w->in_features * 2u < (1ull << 32) &&
         static_cast<uint64_t>(n) * w->in_features / 2u < (1ull << 32) &&
-        static_cast<uint64_t>(m) * n * 2u < (1ull << 32) && mh::aligned(c, 16) && mh::aligned(w->scales, 16) &&
-        mh::aligned(w->biases, 16)) {
+        static_cast<uint64_t>(m) * n * 2u < (1ull << 32) && mh::aligned(c, 16)) {
+        const bool thin = mh::aligned(w->scales, 16) && mh::aligned(w->biases, 16);
         // the segment kernel on 256 x 256 only for long sums with an entry
         // per CU (8192 x 2048 x 11776: 355 us against 366; 4096: 220 / 204)
-        const uint32_t segs = (m + 255u) / 256u * (n / 256u);
-        if (n % 256 == 0 && segs >= 256u && w->in_features > 2048u) {
-            g.dense_bm = 256u;
-            return launch_seg<kSegRBMax, kSegStages, 2, 1, false, EPI_STORE>(g, segs, s);
+        if (thin && !(n % 256 == 0 && segs >= 256u && w->in_features > 2048u)) {
+            return gemm_dense_thin(g, s);
         }
-        return gemm_dense_thin(g, s);
+        // Scales and biases that k_thin's 16-byte register loads cannot take
+        // (the segment kernel's direct-to-LDS loads need 4 bytes): the segment
+        // kernel on 256 x 256 entries, or 128 x 256, whichever first gives one
+        // per CU, else the 128-row tiles below (scales 4 bytes off, us against
+        // those: 4095 x 2048 x 2048 43 / 62, 4095 x 6144 x 2048 116 / 134,
+        // 8192 x 2048 x 11776 326 / 440).
+        if (n % 256 == 0 && segs128 >= 256u && mh::aligned(w->scales, 4) && mh::aligned(w->biases, 4)) {
+            g.dense_bm = segs >= 256u ? 256u : 128u;
+            return launch_seg<kSegRBMax, kSegStages, 2, 1, false, EPI_STORE>(g, segs >= 256u ? segs : segs128, s);
+        }
     }
     const uint32_t mt = (m + 127u) / 128u;
     if (n % 256 == 0) {

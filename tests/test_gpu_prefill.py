@@ -608,3 +608,45 @@ def test_dense_gemm_unaligned_output(dev, orc):
     got = from_dev(c, np.uint16)
     assert not got[:2].any()
     assert_close(got[2:].reshape(m, n), orc.gemm_q4_grouped(a, w, blocks, nb, n, 64), "dense unaligned")
+
+
+def _dev_quant_off(w, off):
+    """dev_quant with scales and biases `off` bytes past a 16-byte boundary."""
+    wd, keep = dev_quant(w)
+    bufs = []
+    for t in (w.scales, w.biases):
+        b = np.zeros(t.size + 64, np.uint16)
+        b[off // 2:off // 2 + t.size] = t.ravel()
+        bufs.append(to_dev(b))
+    return hip.QuantWeights(wd.codes, bufs[0].data_ptr() + off, bufs[1].data_ptr() + off, w.n, w.k, w.group_size,
+                            w.bits), (keep, bufs)
+
+
+@pytest.mark.parametrize("off", [4, 8])
+@pytest.mark.parametrize("m,n,k", [
+    # K in slices; the segment kernel on 128- and on 256-row entries with a
+    # ragged last one; 128-row tiles of 256 and of 64 columns
+    (300, 512, 512), (4100, 2048, 512), (1100, 13312, 512), (700, 2048, 512), (5000, 384, 512)])
+def test_dense_gemm_unaligned_scales(dev, orc, m, n, k, off):
+    """Scales and biases that are 4- or 8-byte aligned: the same bits as
+    16-byte aligned ones (every kernel the dispatch takes without the K slices
+    sums a row in the same k order, and the slices take both), and the oracle's
+    values within the GEMM tolerance."""
+    _log(f"dense {m}x{n}x{k}, scales {off} bytes off")
+    rng = np.random.default_rng(m + n + off)
+    w = layout.synth_quant(rng, n, k, 4)
+    a = layout.synth_bf16(rng, (m, k))
+    ad = to_dev(a)
+    wd, keep = dev_quant(w)
+    c = zeros_dev((m, n), np.uint16)
+    hip.gemm_q4_dense(ad, m, wd, c)
+    want = from_dev(c, np.uint16)
+    wo, keep_o = _dev_quant_off(w, off)
+    c2 = zeros_dev((m, n), np.uint16)
+    hip.gemm_q4_dense(ad, m, wo, c2)
+    got = from_dev(c2, np.uint16)
+    np.testing.assert_array_equal(got, want)
+    rows = np.unique(np.r_[0:40, m // 2:m // 2 + 40, m - 70:m])
+    blocks, nb = _dense_map(len(rows), n)
+    assert_close(got[rows], orc.gemm_q4_grouped(np.ascontiguousarray(a[rows]), w, blocks, nb, n, 64),
+                 f"dense {m}x{n}x{k} off {off}")
