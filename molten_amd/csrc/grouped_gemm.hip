@@ -123,9 +123,12 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void k_grouped(GemmArgs a
         aoffs[q] = src * K * 2u + chunk * 16u;
     }
     // B: this lane's weight row (column) per column block and matrix.  The
-    // scale/bias load is one dword per lane: lanes 0-31 the column's scale
-    // pair (groups kb & ~1, kb | 1), lanes 32-63 its bias pair.
-    uint32_t boffs[NB], sboffs[NB];
+    // scale/bias load is one dword per lane, lanes 0-31 of the scales, 32-63
+    // of the biases: the aligned pair of the whole array that holds the
+    // column's group kb (element sidx + kb).  With an odd number of groups per
+    // row that pair may span two rows; a pair counted from the row's own start
+    // would reach past the array in its last row's last group.
+    uint32_t boffs[NB], sidx[NB];
 #pragma unroll
     for (int cb = 0; cb < NBW; ++cb) {
         const uint32_t col = static_cast<uint32_t>((wave * NBW + cb) * 32 + i32);
@@ -133,7 +136,7 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void k_grouped(GemmArgs a
 #pragma unroll
         for (int mat = 0; mat < NMAT; ++mat) {
             boffs[mat * NBW + cb] = r * (K / 2u) + 16u * h;
-            sboffs[mat * NBW + cb] = r * groups * 2u;
+            sidx[mat * NBW + cb] = r * groups;
         }
     }
 
@@ -150,7 +153,7 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void k_grouped(GemmArgs a
 #pragma unroll
         for (int t = 0; t < NB; ++t) {
             const mh::gbytes sb = h ? bbase[t / NBW] : sbase[t / NBW];
-            dma4(sb + sboffs[t] + (kb & ~1u) * 2u, base + A_BYTES + B_BYTES + (wave * NB + t) * 256u);
+            dma4(sb + ((sidx[t] + kb) & ~1u) * 2u, base + A_BYTES + B_BYTES + (wave * NB + t) * 256u);
         }
     };
 
@@ -207,10 +210,10 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void k_grouped(GemmArgs a
             lgkm_wait<0>(bcode);
             tie_regs(sw);
             tie_regs(bw);
-            const uint32_t half = (kb & 1u) ? 0u : 16u;  // bf16 of group kb in the high half
             float sf[NB], bf[NB];
 #pragma unroll
             for (int t = 0; t < NB; ++t) {
+                const uint32_t half = ((sidx[t] + kb) & 1u) ? 0u : 16u;  // an odd element is its pair's high half
                 sf[t] = __uint_as_float((sw[t] << half) & 0xffff0000u);
                 bf[t] = __uint_as_float((bw[t] << half) & 0xffff0000u);
             }

@@ -650,3 +650,26 @@ def test_dense_gemm_unaligned_scales(dev, orc, m, n, k, off):
     blocks, nb = _dense_map(len(rows), n)
     assert_close(got[rows], orc.gemm_q4_grouped(np.ascontiguousarray(a[rows]), w, blocks, nb, n, 64),
                  f"dense {m}x{n}x{k} off {off}")
+
+
+@pytest.mark.parametrize("m,n,k", [(300, 512, 576), (40, 128, 64), (130, 192, 1600), (5, 64, 192)])
+def test_dense_gemm_odd_groups(dev, orc, m, n, k):
+    """An odd number of groups per row: a column's scale and bias words lie in
+    either half of their pair, by row; one-hot rows reproduce the dequantized
+    columns exactly (the last row's last group among them), random ones match
+    the oracle."""
+    _log(f"dense {m}x{n}x{k}")
+    rng = np.random.default_rng(m + n + k)
+    w = layout.synth_quant(rng, n, k, 4)
+    wd, keep = dev_quant(w)
+    cols = rng.integers(0, k, m)
+    cols[-1] = k - 1
+    a1 = np.zeros((m, k), np.uint16)
+    a1[np.arange(m), cols] = layout.f32_to_bf16(np.float32(1.0))
+    c = zeros_dev((m, n), np.uint16)
+    hip.gemm_q4_dense(to_dev(a1), m, wd, c)
+    np.testing.assert_array_equal(from_dev(c, np.uint16), orc.dequant_bf16(w)[:, cols].T)
+    a = layout.synth_bf16(rng, (m, k))
+    hip.gemm_q4_dense(to_dev(a), m, wd, c)
+    blocks, nb = _dense_map(m, n)
+    assert_close(from_dev(c, np.uint16), orc.gemm_q4_grouped(a, w, blocks, nb, n, 64), f"dense {m}x{n}x{k}")
