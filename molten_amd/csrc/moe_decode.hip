@@ -341,14 +341,20 @@ int launch_router_tiles_as(const DenseArgs& a, hipStream_t stream) {
 
 template <typename WT>
 int launch_router_tiles(const DenseArgs& a, hipStream_t stream) {
-    // smaller tiles while they are what fills the chip (a tile of 64 x 8 is a
-    // chain of ~20 us however few there are): f32 router of 64 experts, step
-    // of 21 255 500 1023 2048 4096 tokens by tile, 64 x 8: 115 134 150 179 250
-    // 390 us; 16 x 8: 103 122 139 169 247 406; 16 x 2: 98 117 139 174 257 421
-    if (a.m <= 512u) {
+    // The smallest tile (tokens x experts) whose workgroups are few rounds of
+    // the chip: a tile of 64 x 8 is a chain of ~17 us however few there are, a
+    // smaller one stages the experts' rows and x more often.  us by workgroups
+    // of the smaller tile, K 2048, 4 to 256 experts, f32 (bf16 the same):
+    // 16 x 2 against 16 x 8: 512 workgroups 5.4 / 7.5, 704 7.3 / 7.5, 800
+    // 8.6 / 7.6, 1024 8.6 / 7.7; 16 x 8 against 64 x 8: 800 15.7 / 19.4, 1024
+    // 16.0 / 18.1, 1280 20.9 / 20.4, 1408 22.3 / 20.8, 2048 29.5 / 21.6.
+    auto tiles = [&](uint32_t tokens, uint32_t experts) {
+        return static_cast<uint64_t>((a.m + tokens - 1u) / tokens) * ((a.n + experts - 1u) / experts);
+    };
+    if (tiles(16u, 2u) <= 768u) {
         return launch_router_tiles_as<WT, 16, 2>(a, stream);
     }
-    if (a.m <= 2048u) {
+    if (tiles(16u, 8u) <= 1024u) {
         return launch_router_tiles_as<WT, 16, 8>(a, stream);
     }
     return launch_router_tiles_as<WT, 64, 8>(a, stream);

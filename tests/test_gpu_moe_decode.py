@@ -272,6 +272,25 @@ def test_prefill_router_and_route_batch(dev, orc):
     np.testing.assert_array_equal(from_dev(gw, np.uint16), want_w)
 
 
+@pytest.mark.parametrize("f32", [True, False])
+@pytest.mark.parametrize("m,e,k", [
+    # tiles of 16 x 2 (odd experts, partial token tiles, the last count of
+    # workgroups that takes them), of 16 x 8 from the next on, of 64 x 8
+    (2, 3, 2048), (17, 17, 512), (512, 33, 1024), (12288, 2, 64), (12289, 2, 64), (700, 64, 2048), (801, 33, 1024),
+    (1025, 61, 2048), (2048, 64, 512), (2049, 64, 512), (1023, 131, 992), (16385, 3, 32)])
+def test_prefill_router_tiles(dev, orc, m, e, k, f32):
+    """Every tile of the prefill router gives the chunk-order logits, bit for bit."""
+    _log(f"router {m}x{e}x{k} {'f32' if f32 else 'bf16'}")
+    rng = np.random.default_rng(m + e + k)
+    w = router_weights(rng, e, k, f32)
+    x = layout.synth_bf16(rng, (m, k))
+    logits = zeros_dev((m + 1, e), np.float32)
+    hip.router_prefill(to_dev(x), to_dev(w), logits, m, k, e)
+    got = from_dev(logits, np.float32)
+    np.testing.assert_array_equal(got[:m], orc.gemv_dense(w, x))
+    assert not got[m].any()  # nothing past the last token
+
+
 @pytest.mark.parametrize("e", [64, 100, 256])
 def test_route_special_values_match_serial_scan(dev, orc, e):
     """NaN and -inf candidates never win, exact ties go to the lower id, and a
