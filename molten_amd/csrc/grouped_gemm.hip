@@ -883,7 +883,7 @@ int dispatch(const GemmArgs& a, uint32_t n_blocks, uint32_t bm, uint32_t bn, hip
                      static_cast<uint64_t>(a.s_rows) * a.n * 2u < (1ull << 32) &&
                      mh::aligned(a.out0, 16) && (a.out1 == nullptr || mh::aligned(a.out1, 16));
     if (a.stamps != nullptr || a.ordered) {  // launch-ordered maps, measurement: the segment kernels only
-        if (seg && thin_fits(a, bn)) {
+        if (seg && thin_fits(a)) {
             if constexpr (EPI == EPI_STORE && !GATHER) {
                 if (bn == 256) return gemm_grouped_thin(a, n_blocks, s);
             } else if constexpr (EPI == EPI_SWIGLU && GATHER) {

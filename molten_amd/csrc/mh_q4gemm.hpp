@@ -30,7 +30,7 @@ struct GemmArgs {
 };
 
 // thin_gemm.hip: launch-ordered products.
-bool thin_fits(const GemmArgs& a, uint32_t bn);
+bool thin_fits(const GemmArgs& a);
 int gemm_gu_act_thin(const GemmArgs& a, uint32_t n_entries, hipStream_t s);
 int gemm_grouped_thin(const GemmArgs& a, uint32_t n_entries, hipStream_t s);
 // thin_gemm.hip: the dense product (n % 128 == 0, k % 512 == 0, the segment

@@ -384,18 +384,19 @@ int launch_dense(GemmArgs g, hipStream_t s) {
 namespace mh {
 
 // Whether these kernels run a launch-ordered product (its offset and
-// alignment limits checked as the segment kernel's).  Scales and biases are
+// alignment limits checked as the segment kernel's): scales and biases are
 // read 16 bytes at a time (make_args leaves the second matrix's null where
-// there is one).  Where every expert has 208 to 288 rows the segment kernel
-// covers each in one pass, and with two workgroups' worth of entries per CU
-// it is level or a little better (64 experts, step of 3500, 3800, 4096 tokens
-// routed evenly: 324 344 373 us against 325 347 378; 3000: 295 against 293;
-// routed unevenly, 4096: 405 against 384).  The host knows only the mean.
-bool thin_fits(const GemmArgs& a, uint32_t bn) {
-    const uint32_t n_experts = a.w_rows / a.n;
-    const bool one_pass = n_experts * (a.n / bn) >= 512u && a.s_rows > 208u * n_experts && a.s_rows <= 288u * n_experts;
-    return a.ordered && a.stamps == nullptr && !one_pass && aligned(a.s0, 16) && aligned(a.b0, 16) &&
-           aligned(a.s1, 16) && aligned(a.b1, 16);
+// there is one).  The segment kernel covers an expert of up to 288 rows in
+// one pass and dequantizes its codes once, but is level at best.  Steps with
+// 208 to 288 rows per expert in the mean, us on the segment kernel against
+// these: routed evenly, 64 experts of 2048 x 1536 368 to 424 / 378 to 424
+// (4096 tokens, by box and load: 4% faster to 3% slower), 128 experts 800 /
+// 780, 48 experts 306 / 271 (2.25 rounds of its workgroups); unevenly (a
+// selection bias), 64 experts 412 to 453 / 385 to 423, 128 experts 883 / 791,
+// 256 experts of 1024 x 512 519 / 468.  The host knows only the mean.
+bool thin_fits(const GemmArgs& a) {
+    return a.ordered && a.stamps == nullptr && aligned(a.s0, 16) && aligned(a.b0, 16) && aligned(a.s1, 16) &&
+           aligned(a.b1, 16);
 }
 
 template <int NBW, int NMAT, bool GATHER, int EPI>

@@ -512,7 +512,9 @@ def test_dense_gemm_segment_path(dev, orc, m, n, k):
     (64, 512, 512, 60, True), (64, 1536, 512, 300, True), (16, 512, 1024, 1000, True),
     # column tiles in groups (4, 8, 16 and 24 of them), ragged last passes
     (16, 1024, 512, 128, False), (64, 2048, 1024, 1025, False), (24, 512, 1536, 700, False),
-    (64, 2048, 1024, 2304, False)])
+    (64, 2048, 1024, 2304, False),
+    # 208 to 288 rows per expert in the mean, uneven and with an expert of all tokens
+    (64, 2048, 1024, 3700, False), (64, 2048, 1024, 4095, True)])
 def test_moe_prefill_matches_segment_kernel(dev, e, h, inter, m, skewed):
     """The step's grouped GEMMs against the segment kernel's (the stamped step
     runs that one): the
