@@ -946,6 +946,7 @@ GemmArgs make_args(const uint16_t* a, const uint32_t* gather, uint32_t a_rows,
     g.s_rows = s_rows;
     g.a_rows = a_rows;
     g.w_rows = w0->out_features;
+    g.expert_rows = s_rows;
     return g;
 }
 
@@ -955,23 +956,26 @@ namespace mh {
 
 // The prefill step's two grouped GEMMs (as mh_gemm_q4_grouped_gu_act and
 // mh_gemm_q4_grouped, the segment kernels only): on a launch-ordered map
-// (n_blocks: its map_grid entries) and / or with workgroup stamps.
+// (n_blocks: its map_grid entries) and / or with workgroup stamps; no expert
+// has more than expert_rows rows.
 int gemm_gu_act_seg(const uint16_t* x, const uint32_t* ids_sorted, uint32_t x_rows, const mh_quant_weights* gate,
                     const mh_quant_weights* up, uint16_t* act, const uint32_t* blocks, uint32_t n_blocks,
-                    uint32_t s_rows, uint32_t n, uint32_t bm, uint32_t bn, bool ordered, uint64_t* stamps,
-                    hipStream_t s) {
+                    uint32_t s_rows, uint32_t n, uint32_t bm, uint32_t bn, bool ordered, uint32_t expert_rows,
+                    uint64_t* stamps, hipStream_t s) {
     GemmArgs g = make_args(x, ids_sorted, x_rows, gate, up, act, nullptr, blocks, s_rows, n);
     g.ordered = ordered ? 1u : 0u;
     g.stamps = stamps;
+    g.expert_rows = expert_rows;
     return dispatch<true, EPI_SWIGLU>(g, n_blocks, bm, bn, s);
 }
 
 int gemm_grouped_seg(const uint16_t* a, const mh_quant_weights* w, uint16_t* c, const uint32_t* blocks,
                      uint32_t n_blocks, uint32_t s_rows, uint32_t n, uint32_t bm, uint32_t bn, bool ordered,
-                     uint64_t* stamps, hipStream_t s) {
+                     uint32_t expert_rows, uint64_t* stamps, hipStream_t s) {
     GemmArgs g = make_args(a, nullptr, s_rows, w, nullptr, c, nullptr, blocks, s_rows, n);
     g.ordered = ordered ? 1u : 0u;
     g.stamps = stamps;
+    g.expert_rows = expert_rows;
     return dispatch<false, EPI_STORE>(g, n_blocks, bm, bn, s);
 }
 
@@ -1082,7 +1086,8 @@ int mh_gemm_q4_grouped_ordered(const uint16_t* a, const mh_quant_weights* w, uin
     MH_TRY(gemm_checks(op, a, w, c, ord, n_entries, s_rows, n));
     MH_ENSURE(bn == 256u && n % bn == 0u, MH_ERR_UNSUPPORTED, "%s: tile width %u (256 only)", op, bn);
     MH_TRY(ordered_checks(op, n_entries, n, bn));
-    return mh::gemm_grouped_seg(a, w, c, ord, n_entries, s_rows, n, bm, bn, true, nullptr, mh::as_stream(stream));
+    return mh::gemm_grouped_seg(a, w, c, ord, n_entries, s_rows, n, bm, bn, true, s_rows, nullptr,
+                                mh::as_stream(stream));
 }
 
 int mh_gemm_q4_grouped_gu_act_ordered(const uint16_t* x, const uint32_t* ids_sorted, uint32_t x_rows,
@@ -1099,7 +1104,7 @@ int mh_gemm_q4_grouped_gu_act_ordered(const uint16_t* x, const uint32_t* ids_sor
     MH_ENSURE(bn == 128u && n % bn == 0u, MH_ERR_UNSUPPORTED, "%s: tile width %u (128 only)", op, bn);
     MH_TRY(ordered_checks(op, n_entries, n, bn));
     return mh::gemm_gu_act_seg(x, ids_sorted, x_rows, gate, up, act, ord, n_entries, s_rows, n, bm, bn, true,
-                               nullptr, mh::as_stream(stream));
+                               s_rows, nullptr, mh::as_stream(stream));
 }
 
 }  // extern "C"

@@ -105,17 +105,20 @@ int moe_decode_fused(const void* router, int router_dtype, const float* bias, in
 // Workgroups x waves of the fused decode step (the stamp buffer holds
 // kGrid * kWaves * MH_MOE_DECODE_STAMPS words).
 uint32_t moe_decode_fused_waves();
-// The prefill step's grouped GEMMs on the segment kernels (grouped_gemm.hip):
-// ordered, the map is in launch order (entry b for workgroup b, map_grid
-// entries, from moe_route_sort_maps' gu_ord / dn_ord); stamps (or null), per
-// workgroup MH_PREFILL_STAMPS words (measurement).
+// The prefill step's grouped GEMMs (grouped_gemm.hip): ordered, the map is in
+// launch order (map_grid entries, from moe_route_sort_maps' gu_ord / dn_ord),
+// run by k_thin (thin_gemm.hip), or by the segment kernel (entry b for
+// workgroup b) where thin_fits does not hold; stamps (or null), the segment
+// kernel with MH_PREFILL_STAMPS words per workgroup (measurement).  expert_rows:
+// the rows an expert has at most, for the launch's size (an expert with more is
+// only slower).
 int gemm_gu_act_seg(const uint16_t* x, const uint32_t* ids_sorted, uint32_t x_rows, const mh_quant_weights* gate,
                     const mh_quant_weights* up, uint16_t* act, const uint32_t* blocks, uint32_t n_blocks,
-                    uint32_t s_rows, uint32_t n, uint32_t bm, uint32_t bn, bool ordered, uint64_t* stamps,
-                    hipStream_t s);
+                    uint32_t s_rows, uint32_t n, uint32_t bm, uint32_t bn, bool ordered, uint32_t expert_rows,
+                    uint64_t* stamps, hipStream_t s);
 int gemm_grouped_seg(const uint16_t* a, const mh_quant_weights* w, uint16_t* c, const uint32_t* blocks,
                      uint32_t n_blocks, uint32_t s_rows, uint32_t n, uint32_t bm, uint32_t bn, bool ordered,
-                     uint64_t* stamps, hipStream_t s);
+                     uint32_t expert_rows, uint64_t* stamps, hipStream_t s);
 // stamps: per-wave phase timestamps (measurement, batch 8 only), or null.
 int gemv_mfma(const mh_quant_weights* w, const uint16_t* x, uint16_t* y, uint64_t* slots, uint32_t* ids,
               uint32_t batch, hipStream_t stream, uint64_t* stamps = nullptr);

@@ -22,6 +22,7 @@ struct GemmArgs {
     uint16_t* out1;          // [s_rows, n]: up (EPI_GATE_UP)
     const uint4* blocks;     // block map; null: a dense product (entries computed)
     uint32_t k, n, s_rows, a_rows, w_rows;
+    uint32_t expert_rows;    // k_thin: rows an expert is taken to have at most (sizes its parts)
     uint32_t dense_bm;       // rows per entry of a dense product
     uint32_t parts;          // k_thin: workgroups per map entry (its passes dealt out in turn)
     uint32_t part_units;     // k_thin: map rows whose parts are launched part by part

@@ -17,7 +17,7 @@
 
 namespace {
 
-constexpr uint32_t kBM = 512;      // row tile of both grouped GEMMs (segment kernels)
+constexpr uint32_t kBM = 512;      // rows per entry of both grouped GEMMs' maps (one expert's)
 constexpr uint32_t kGuBN = 128;    // gate/up tile width (fused SwiGLU)
 constexpr uint32_t kDnBN = 256;    // down tile width
 
@@ -158,9 +158,10 @@ int prefill(const char* op, const void* router, int router_dtype, const float* b
         // ranking; thin_gemm.hip), or the segment kernels stamped
         const hipStream_t hs = mh::as_stream(stream);
         MH_TRY(mh::gemm_gu_act_seg(x, ids_sorted, m, gate, up, act, l.ordered ? gu_ord : gu_map,
-                                   l.ordered ? l.grid_gu : l.max_gu, s, n_inter, kBM, kGuBN, l.ordered, stamps, hs));
+                                   l.ordered ? l.grid_gu : l.max_gu, s, n_inter, kBM, kGuBN, l.ordered, m, stamps,
+                                   hs));
         MH_TRY(mh::gemm_grouped_seg(act, down, ed, l.ordered ? dn_ord : dn_map, l.ordered ? l.grid_dn : l.max_dn, s,
-                                    d_model, kBM, kDnBN, l.ordered,
+                                    d_model, kBM, kDnBN, l.ordered, m,
                                     stamps != nullptr ? stamps + static_cast<size_t>(MH_PREFILL_STAMP_WGS) *
                                                                      MH_PREFILL_STAMPS
                                                       : nullptr,

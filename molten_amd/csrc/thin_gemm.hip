@@ -20,6 +20,8 @@
 // (4.1 TB/s; the segment kernel 94 + 50); with dequant and MFMAs taken out the
 // loads alone take 50 + 26.  Dense 4095 x 6144 x 2048: 100 us (1030 TFLOP/s;
 // the segment kernel 118), 1023 x 6144 x 2048 35 (60).
+#include <algorithm>
+
 #include "mh_device.hpp"
 #include "mh_host.hpp"
 #include "mh_q4gemm.hpp"
@@ -401,15 +403,22 @@ bool thin_fits(const GemmArgs& a) {
 
 template <int NBW, int NMAT, bool GATHER, int EPI>
 static int launch_grouped(GemmArgs g, uint32_t n_entries, uint32_t n_experts, hipStream_t s) {
-    // One row block per pass needs less LDS (three workgroups per CU), but an
-    // expert of more than 32 rows takes several passes then: up to a mean of 4
-    // rows (64 experts top-4: 60 tokens 135.6 us against 138.1).
+    // One row block per pass needs less LDS (three workgroups per CU): up to a
+    // mean of 4 rows (step of 64 experts of 2048 x 1536 top-4, 64 tokens 97 us
+    // against 102; 256 experts of 2048 x 512, 255 tokens 118 / 129).  An expert
+    // that many tokens choose takes several passes then, dealt out to
+    // up to four workgroups: 64 experts top-2, 128 tokens, one expert chosen by
+    // all 149 -> 96 us, 256 experts top-4, 255 tokens 228 -> 152.  The first parts of all entries are
+    // launched before the others, most of which have no pass: in groups as
+    // below those take places among the live ones (64 tokens, no such expert,
+    // 97 us with one part, 98 so, 105 in groups).
     const uint32_t nt = g.n / (kThinWaves * NBW * 32u);
-    g.part_units = (32u + nt - 1u) / nt;
     if (g.s_rows <= 4u * n_experts) {
-        g.parts = 1u;
+        g.parts = std::min(4u, (g.expert_rows + 31u) / 32u);
+        g.part_units = n_entries / (8u * nt);
         return launch_thin<1, NBW, NMAT, GATHER, EPI>(g, n_entries, s);
     }
+    g.part_units = (32u + nt - 1u) / nt;
     // a workgroup for every pass of a 512-row entry (step of 255, 1023, 2048,
     // 4096 tokens: 133 178 242 392 us; one workgroup per entry 135 187 266
     // 422, the segment kernel 185 213 285 408)

@@ -510,6 +510,8 @@ def test_dense_gemm_segment_path(dev, orc, m, n, k):
     (64, 512, 512, 1, False), (64, 512, 512, 33, False), (64, 512, 512, 64, False), (64, 512, 512, 65, False),
     # an expert with every token: two passes of one row block, three and eight of four
     (64, 512, 512, 60, True), (64, 1536, 512, 300, True), (16, 512, 1024, 1000, True),
+    # in passes of one row block: three, and eight on four workgroups
+    (256, 1024, 512, 96, True), (256, 512, 512, 250, True),
     # column tiles in groups (4, 8, 16 and 24 of them), ragged last passes
     (16, 1024, 512, 128, False), (64, 2048, 1024, 1025, False), (24, 512, 1536, 700, False),
     (64, 2048, 1024, 2304, False),
