@@ -559,6 +559,8 @@ def test_moe_prefill_matches_segment_kernel(dev, e, h, inter, m, skewed):
     # K cut into slices: one row, empty slices (k 128: one block for 8 waves), ragged
     # rows and blocks, 64-row and 128-row tiles, many columns on few slices
     (1, 64, 128), (33, 576, 384), (32, 11776, 256), (21, 512, 11776), (300, 2048, 640), (500, 2048, 512), (60, 9216, 256),
+    # the tallest in slices, and past it
+    (12288, 64, 256), (12289, 64, 256),
     # column tiles of 128 and 256, one workgroup per CU up to many, scales past 2048 k
     (257, 6144, 512), (700, 2048, 4608), (4100, 2048, 512), (4100, 6144, 512)])
 def test_dense_gemm_small_and_wide_tiles(dev, orc, m, n, k):
