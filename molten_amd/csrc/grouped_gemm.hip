@@ -1009,14 +1009,14 @@ int mh_gemm_q4_dense(const uint16_t* a, uint32_t m, const mh_quant_weights* w, u
     if (gemm_dense_slices(a, m, w, c, s, &rc)) {
         return rc;
     }
-    const uint32_t segs = (m + 255u) / 256u * (n / 256u), segs128 = (m + 127u) / 128u * (n / 256u);
     if (n % 128 == 0 && w->in_features % 512u == 0 && static_cast<uint64_t>(m) * w->in_features * 2u < (1ull << 32) &&
         static_cast<uint64_t>(n) * w->in_features / 2u < (1ull << 32) &&
         static_cast<uint64_t>(m) * n * 2u < (1ull << 32) && mh::aligned(c, 16)) {
-        const bool thin = mh::aligned(w->scales, 16) && mh::aligned(w->biases, 16);
-        // the segment kernel on 256 x 256 only for long sums with an entry
-        // per CU (8192 x 2048 x 11776: 355 us against 366; 4096: 220 / 204)
-        if (thin && !(n % 256 == 0 && segs >= 256u && w->in_features > 2048u)) {
+        // (the segment kernel on 256 x 256 is 1 to 4% faster where its entries
+        // make whole rounds of the chip and K is long, up to 30% slower between:
+        // 8192 x 2048 x 11776 334 us against 344, 9000 573 / 461, 12000 640 /
+        // 518; 4095 x 6144 x 4096 220 / 185)
+        if (mh::aligned(w->scales, 16) && mh::aligned(w->biases, 16)) {
             return gemm_dense_thin(g, s);
         }
         // Scales and biases that k_thin's 16-byte register loads cannot take
@@ -1025,6 +1025,7 @@ int mh_gemm_q4_dense(const uint16_t* a, uint32_t m, const mh_quant_weights* w, u
         // per CU, else the 128-row tiles below (scales 4 bytes off, us against
         // those: 4095 x 2048 x 2048 43 / 62, 4095 x 6144 x 2048 116 / 134,
         // 8192 x 2048 x 11776 326 / 440).
+        const uint32_t segs = (m + 255u) / 256u * (n / 256u), segs128 = (m + 127u) / 128u * (n / 256u);
         if (n % 256 == 0 && segs128 >= 256u && mh::aligned(w->scales, 4) && mh::aligned(w->biases, 4)) {
             g.dense_bm = segs >= 256u ? 256u : 128u;
             return launch_seg<kSegRBMax, kSegStages, 2, 1, false, EPI_STORE>(g, segs >= 256u ? segs : segs128, s);

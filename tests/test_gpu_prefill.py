@@ -479,10 +479,10 @@ def test_dense_gemm_one_hot_is_exact_dequant(dev, orc):
 
 @pytest.mark.parametrize("m,n,k", [(1100, 13312, 512), (1100, 7936, 512)])
 def test_dense_gemm_segment_path(dev, orc, m, n, k):
-    """Shapes with >= 256 segment entries of 256 x 256 (13312 columns: 5 row
-    segments, the last of 76 rows, x 52 column tiles) or, below that, of
-    128 x 256 (7936 columns: 9 row segments, the last of 76 rows, x 31): the
-    segment kernel in dense mode.  One-hot rows reproduce the dequantized
+    """Wide shapes (13312 columns: 9 row tiles of 128, the last of 76 rows, x 52
+    column tiles of 256; 7936 columns: x 31), on k_thin's widest tiles: the
+    segment kernel takes them only with scales that are not 16-byte aligned
+    (test_dense_gemm_unaligned_scales).  One-hot rows reproduce the dequantized
     columns exactly over every tile, and the first and the last (partial)
     row segments match the oracle within tolerance."""
     rng = np.random.default_rng(11)
@@ -562,7 +562,9 @@ def test_moe_prefill_matches_segment_kernel(dev, e, h, inter, m, skewed):
     # the tallest in slices, and past it
     (12288, 64, 256), (12289, 64, 256),
     # column tiles of 128 and 256, one workgroup per CU up to many, scales past 2048 k
-    (257, 6144, 512), (700, 2048, 4608), (4100, 2048, 512), (4100, 6144, 512)])
+    (257, 6144, 512), (700, 2048, 4608), (4100, 2048, 512), (4100, 6144, 512), (2100, 6144, 2560),
+    # neither slices nor 512 k a scale block: 128-row tiles of 256 and of 64 columns
+    (1500, 2048, 640), (2000, 576, 640)])
 def test_dense_gemm_small_and_wide_tiles(dev, orc, m, n, k):
     """Every tile of the dense product: one-hot rows reproduce the dequantized
     columns exactly, and the first rows, a middle run and the last (partial)
@@ -588,7 +590,7 @@ def test_dense_gemm_small_and_wide_tiles(dev, orc, m, n, k):
 
 
 def test_dense_gemm_segment_kernel_long_sums(dev, orc):
-    """K past 2048 with a 256 x 256 entry per CU: the segment kernel."""
+    """K past 2048 with a 256 x 256 tile per CU."""
     m, n, k = 8100, 2048, 2560
     rng = np.random.default_rng(5)
     w = layout.synth_quant(rng, n, k, 4)
@@ -632,7 +634,9 @@ def _dev_quant_off(w, off):
 @pytest.mark.parametrize("m,n,k", [
     # K in slices; the segment kernel on 128- and on 256-row entries with a
     # ragged last one; 128-row tiles of 256 and of 64 columns
-    (300, 512, 512), (4100, 2048, 512), (1100, 13312, 512), (700, 2048, 512), (5000, 384, 512)])
+    (300, 512, 512), (4100, 2048, 512), (1100, 13312, 512), (700, 2048, 512), (5000, 384, 512),
+    # sums past 2048 k on the segment kernel
+    (1100, 7936, 2560), (1100, 13312, 2560)])
 def test_dense_gemm_unaligned_scales(dev, orc, m, n, k, off):
     """Scales and biases that are 4- or 8-byte aligned: the same bits as
     16-byte aligned ones (every kernel the dispatch takes without the K slices
