@@ -62,6 +62,33 @@ __device__ __forceinline__ void dma16s(mh::gbytes base, uint32_t voff, uint32_t 
         : "v"(voff), "s"(base), "s"(lds_base)
         : "memory");
 }
+// dma16s to LDS address lds_base + OFF + 16 l, M0 written and not restored.  The
+// clobber makes the compiler set M0 again before a use of its own (its warning
+// is that it will not save a reserved register's old value).
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+template <int OFF>
+__device__ __forceinline__ void dma16m(mh::gbytes base, uint32_t voff, uint32_t lds_base) {
+    asm volatile(
+        "s_add_u32 m0, %2, %3\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %0, %1"
+        :
+        : "v"(voff), "s"(base), "s"(lds_base), "n"(OFF)
+        : "memory", "scc", "m0");
+}
+// The same with 4 bytes per lane and 64-bit lane addresses.
+template <int OFF>
+__device__ __forceinline__ void dma4v(mh::gbytes src, uint32_t lds_base) {
+    asm volatile(
+        "s_add_u32 m0, %1, %2\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dword %0, off"
+        :
+        : "v"(src), "s"(lds_base), "n"(OFF)
+        : "memory", "scc", "m0");
+}
+#pragma clang diagnostic pop
 // Direct-to-LDS 4-byte load: lane l's dword lands at lds_base + 4 l.
 __device__ __forceinline__ void dma4(mh::gbytes src, uint32_t lds_base) {
     __builtin_amdgcn_global_load_lds((glb_ptr)src, (lds_ptr)(uintptr_t)lds_base, 4, 0, 0);

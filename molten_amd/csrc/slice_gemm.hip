@@ -17,30 +17,6 @@ namespace {
 
 using namespace mh;
 
-// Direct-to-LDS loads (global_load_lds) to LDS address lds_base + OFF + 16 (4)
-// bytes per lane; M0 is written and not restored: nothing else in this kernel
-// uses it.
-template <int OFF>
-__device__ __forceinline__ void dma16m(gbytes base, uint32_t voff, uint32_t lds_base) {
-    asm volatile(
-        "s_add_u32 m0, %2, %3\n\t"
-        "s_nop 0\n\t"
-        "global_load_lds_dwordx4 %0, %1"
-        :
-        : "v"(voff), "s"(base), "s"(lds_base), "n"(OFF)
-        : "memory", "scc");
-}
-template <int OFF>
-__device__ __forceinline__ void dma4v(gbytes src, uint32_t lds_base) {
-    asm volatile(
-        "s_add_u32 m0, %1, %2\n\t"
-        "s_nop 0\n\t"
-        "global_load_lds_dword %0, off"
-        :
-        : "v"(src), "s"(lds_base), "n"(OFF)
-        : "memory", "scc");
-}
-
 struct SliceArgs {
     const uint16_t* a;  // [m, k]
     const uint32_t* codes;

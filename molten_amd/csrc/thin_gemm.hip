@@ -33,19 +33,6 @@ using namespace mh;
 constexpr int kThinWaves = 4;
 constexpr int kThinJ = 4;  // scale blocks of 512 k held in registers
 
-// dma16s (mh_mfma.hpp) to LDS address lds_base + OFF, M0
-// written and not restored: nothing else in these kernels uses M0 (every load
-// to the LDS is this one).
-template <int OFF>
-__device__ __forceinline__ void dma16m(gbytes base, uint32_t voff, uint32_t lds_base) {
-    asm volatile(
-        "s_add_u32 m0, %2, %3\n\t"
-        "s_nop 0\n\t"
-        "global_load_lds_dwordx4 %0, %1"
-        :
-        : "v"(voff), "s"(base), "s"(lds_base), "n"(OFF)
-        : "memory", "scc");
-}
 // LDS of a workgroup: A in NSA slots of 64 k, and per wave two slots of B
 // codes (128 k of NB column blocks).
 template <int RBMAX, int NB>
