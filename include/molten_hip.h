@@ -483,9 +483,19 @@ int mh_gemm_quant_bf16_nt(const uint16_t* a, uint32_t m, const mh_quant_weights*
 
 /* src/lfm.rs:661-671 project (prefill): dequant_q4_bf16_bulk + gemm_bf16_nt
  * fused: C[m, :] = A[m, :] . dequant(W)^T for every row m < M, A bf16 [M, K]
- * (16-byte aligned), W 4-bit group 64 [N, K], C bf16 [M, N]; the grouped
- * GEMM's kernel (bf16 dequant, f32 MFMA accumulation) over a dense tiling
- * (128 x 256 tiles, 128 x 64 when N % 256 != 0).  N a multiple of 64. */
+ * (16-byte aligned), W 4-bit group 64 [N, K], C bf16 [M, N] (4-byte aligned);
+ * bf16 dequant, f32 MFMA accumulation.  N a multiple of 64, K of 64.
+ *
+ * Kernels by shape: while tiles of at most 128 rows x 32 columns are few (and
+ * M <= 12288, K a multiple of 128, C 8-byte aligned), such tiles with K cut
+ * into 4 or 8 slices; else, N a multiple of 128 and K of 512, C, scales and
+ * biases 16-byte aligned, tiles of 64 x 128 to 128 x 256; else the grouped
+ * GEMM's kernels over a dense tiling (fastest with scales and biases at least
+ * 4-byte aligned).  The slices are f32 sums of their own, added in slice order;
+ * every other kernel sums a row in one chain over k, the same in all.  So the
+ * f32 summation order of a row, and with it the last bit of some outputs,
+ * depends on (M, N, K): the same prompt row in a chunk of another length may
+ * round differently. */
 int mh_gemm_q4_dense(const uint16_t* a, uint32_t m, const mh_quant_weights* w, uint16_t* c,
                      mh_stream_t stream);
 
@@ -508,10 +518,11 @@ int mh_gemm_q4_grouped_gu_act(const uint16_t* x, const uint32_t* ids_sorted, uin
 
 /* No reference counterpart: the two grouped GEMMs above on a block map in
  * launch order, for callers that hold one (mh_moe_prefill's workspace regions
- * MH_PREFILL_WS_GU_ORD / DN_ORD): entry b is workgroup b's, the map holds a
- * whole number of 8 x (n / bn) entries, all-zero entries for workgroups
- * without one.  Each workgroup reads its entry with one load instead of
- * ranking the map's rows.  Segment tiles only: bm 256 or 512 (rows per
+ * MH_PREFILL_WS_GU_ORD / DN_ORD): entries in the order they are launched in,
+ * a whole number of 8 x (n / bn) of them, all-zero ones where there is none.
+ * A workgroup reads its entry with one load instead of ranking the map's
+ * rows; up to four workgroups share an entry's rows (one with scales or biases
+ * that are not 16-byte aligned).  Segment tiles only: bm 256 or 512 (rows per
  * entry), bn 256 (down) or 128 (gate/up + SwiGLU, with ids_sorted); K a
  * multiple of 512.  Same outputs as the reference-order calls over the same
  * entries. */
@@ -554,7 +565,9 @@ int mh_moe_prefill(const void* router, int router_dtype, const float* bias, int 
 
 /* Measurement only (no reference counterpart): mh_moe_prefill with the two
  * grouped GEMMs on the segment kernel, stamped per workgroup (mh_moe_prefill
- * itself runs tiles of 128 rows; same bits).  `stamps` holds 2 x
+ * itself runs passes of at most 128 rows, 32 with few rows per expert, unless
+ * an expert matrix's scales or biases are not 16-byte aligned or the maps are
+ * too large for the launch order; same bits).  `stamps` holds 2 x
  * MH_PREFILL_STAMP_WGS x MH_PREFILL_STAMPS u64 words (gate/up + SwiGLU, then
  * down); workgroup g of a GEMM writes at g * MH_PREFILL_STAMPS: the 100 MHz
  * constant clock at its start (word 0) and at its end (after its last stores

@@ -882,7 +882,7 @@ int dispatch(const GemmArgs& a, uint32_t n_blocks, uint32_t bm, uint32_t bn, hip
                      static_cast<uint64_t>(a.w_rows) * a.k / 2u < (1ull << 32) &&
                      static_cast<uint64_t>(a.s_rows) * a.n * 2u < (1ull << 32) &&
                      mh::aligned(a.out0, 16) && (a.out1 == nullptr || mh::aligned(a.out1, 16));
-    if (a.stamps != nullptr || a.ordered) {  // launch-ordered maps, measurement: the segment kernels only
+    if (a.stamps != nullptr || a.ordered) {  // launch-ordered maps: k_thin; those it does not take, measurement: k_seg
         if (seg && thin_fits(a)) {
             if constexpr (EPI == EPI_STORE && !GATHER) {
                 if (bn == 256) return gemm_grouped_thin(a, n_blocks, s);
@@ -955,9 +955,8 @@ GemmArgs make_args(const uint16_t* a, const uint32_t* gather, uint32_t a_rows,
 namespace mh {
 
 // The prefill step's two grouped GEMMs (as mh_gemm_q4_grouped_gu_act and
-// mh_gemm_q4_grouped, the segment kernels only): on a launch-ordered map
-// (n_blocks: its map_grid entries) and / or with workgroup stamps; no expert
-// has more than expert_rows rows.
+// mh_gemm_q4_grouped, segment tiles): on a launch-ordered map (n_blocks: its
+// map_grid entries) and / or with workgroup stamps (see mh_host.hpp).
 int gemm_gu_act_seg(const uint16_t* x, const uint32_t* ids_sorted, uint32_t x_rows, const mh_quant_weights* gate,
                     const mh_quant_weights* up, uint16_t* act, const uint32_t* blocks, uint32_t n_blocks,
                     uint32_t s_rows, uint32_t n, uint32_t bm, uint32_t bn, bool ordered, uint32_t expert_rows,
@@ -1072,8 +1071,8 @@ int mh_gemm_q4_grouped_gu_act(const uint16_t* x, const uint32_t* ids_sorted, uin
                       : dispatch<false, EPI_SWIGLU>(g, n_blocks, bm, bn, s);
 }
 
-// The launch-ordered forms: entry b of the map is workgroup b's (a whole
-// number of 8 x (n / bn) units), segment tiles only.
+// The launch-ordered forms: the map's entries in launch order (a whole number
+// of 8 x (n / bn) units), segment tiles only.
 static int ordered_checks(const char* op, uint32_t n_entries, uint32_t n, uint32_t bn) {
     MH_ENSURE(n_entries % (8u * (n / bn)) == 0u, MH_ERR_INVALID,
               "%s: a launch-ordered map holds whole units of 8 x %u entries, not %u", op, n / bn, n_entries);

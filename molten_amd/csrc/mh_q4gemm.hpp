@@ -38,7 +38,7 @@ int gemm_grouped_thin(const GemmArgs& a, uint32_t n_entries, hipStream_t s);
 // kernel's offset and alignment limits).
 int gemm_dense_thin(const GemmArgs& a, hipStream_t s);
 // slice_gemm.hip: the dense product with few output tiles; false where its
-// shape or size is not taken.
+// shape, size or alignment is not taken.
 bool gemm_dense_slices(const uint16_t* a, uint32_t m, const mh_quant_weights* w, uint16_t* c, hipStream_t s, int* rc);
 
 // One Q4 word (8 codes, low nibble first) -> bf16(fma(s, q, b)) x 8.  A code

@@ -5,7 +5,7 @@
 // each a serial chain over the whole K: 58 us for 2.1 GFLOP.  Here a tile is
 // 32 RB rows x 32 columns and its K is cut into KS slices, one per wave of
 // the workgroup, so that the product fills the chip (256 workgroups of 8
-// waves) and a wave's chain is 256 k: 8.5 us, half of it the launch and the
+// waves) and a wave's chain is 256 k: 7.4 us, half of it the launch and the
 // first loads.  What bounds it then is A, which every 32 columns read again
 // from the L2 (64 MB here, about 15 TB/s); from a few hundred workgroups on
 // thin_gemm.hip's wider tiles are the better ones.
@@ -179,11 +179,15 @@ int launch_slice(SliceArgs a, hipStream_t s) {
 namespace mh {
 
 // The smallest tile that keeps one workgroup per CU (us at K 2048 / 11776 by
-// tile: 32 rows 8 slices, 64 rows 8, 64 rows 4, 128 rows 4): 21 x 2048 rows
-// and columns 8.7 8.7 8.8 8.8 (the call's own cost) / 21 25 26 33; 255 x 2048
-// 10.3 9.1 8.9 9.7 / 49 31 33 44; 500 x 2048 18.8 13.2 12.1 10.7; 100 x 6144
-// 14.3 12.2 10.4 9.7; 60 x 11776 14.8 13.3 11.4 17.0.  Past that (255 x 6144:
-// 27 19 16 18) the 64 x 128 tiles of thin_gemm.hip take 15.
+// tile, in a graph: 32 rows 8 slices, 64 rows 8, 64 rows 4, 128 rows 4; then
+// the tiles of thin_gemm.hip): 21 x 2048 rows and columns 5.1 6.4 6.3 8.7, 12.5
+// / 14 20 22 30, 59; 255 x 2048 9.8 7.4 7.1 9.6, 14.0 / 50 35 36 45, 72; 500 x
+// 2048 17.9 13.0 11.7 10.6, 14.3; 100 x 6144 13.4 11.9 10.5 9.7, 14.6; 60 x
+// 11776 13.5 12.3 10.6 16.3, 14.1.  Past that (255 x 6144: 25.7 19.3 16.1 17.6)
+// those take 16.0.
+//
+// The slices are summed apart, 8 or 4 by the tile, so a row's f32 sum runs in
+// another order than on the kernels without them: its bits follow m and n.
 bool gemm_dense_slices(const uint16_t* a, uint32_t m, const mh_quant_weights* w, uint16_t* c, hipStream_t s, int* rc) {
     const uint32_t n = w->out_features, k = w->in_features;
     // 128-k blocks, 32-bit byte offsets, 8-byte stores and whole code pieces; no

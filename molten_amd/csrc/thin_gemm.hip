@@ -12,14 +12,13 @@
 // workgroups per CU (three with one row block), whose loads, dequant and
 // MFMAs cover each other.  That pays for dequantizing an expert's codes once
 // per 128 rows instead of once per 288.  A column's scales and biases are read
-// once, whole, into registers (16 bytes at a time from rows of 64, as the
-// segment kernel's LDS blocks take them, each line was fetched up to four
-// times: 310 MB instead of 235 for gate/up of 64 experts).
+// whole into registers, 64 bytes of a row at a time.
 //
-// Gate/up and down of 64 experts (2048 x 1536, top-4), 100 tokens: 55 + 30 us
-// (4.1 TB/s; the segment kernel 94 + 50); with dequant and MFMAs taken out the
-// loads alone take 50 + 26.  Dense 4095 x 6144 x 2048: 100 us (1030 TFLOP/s;
-// the segment kernel 118), 1023 x 6144 x 2048 35 (60).
+// Gate/up and down of 64 experts (2048 x 1536, top-4), 100 tokens: 57.6 + 31.0
+// us, 215 + 108 MB fetched (the segment kernel 97 + 50 us, 225 + 112 MB); 4096
+// tokens 220 + 117 us at best, 593 + 296 MB (225 + 126 us, 367 + 184 MB): the
+// passes of an expert fetch its codes again.  Dense 4095 x 6144 x 2048: 93 us
+// (1110 TFLOP/s; the segment kernel 116), 1023 x 6144 x 2048 35 (60).
 #include <algorithm>
 
 #include "mh_device.hpp"
@@ -422,10 +421,11 @@ int gemm_grouped_thin(const GemmArgs& a, uint32_t n_entries, hipStream_t s) {
 }
 
 // The dense product: the smallest tile that keeps one workgroup per CU, then
-// the widest (rows x columns of 64 x 128, 128 x 128, 128 x 256; us at K
-// 2048): 255 x 6144 15.3 17.5 29.3; 1023 x 2048 16.0 17.8 29.4; 1023 x 6144
-// 36.6 35.1 35.6; 2047 x 6144 64.6 56.4 60.3; 4095 x 6144 122 106.6 99.8;
-// 4095 x 11776 230 203 185.
+// the widest (rows x columns of 64 x 128, 128 x 128, 128 x 256; us at K 2048,
+// one box, in a graph): 255 x 6144 15.7 20.2 27.2; 1023 x 2048 16.1 19.3 27.4;
+// 400 x 6144 23.3 21.1 29.0; 1023 x 6144 38.7 36.5 35.3; 2047 x 6144 71.6 61.4
+// 61.5; 4095 x 2048 50.3 42.3 40.9; 4095 x 6144 141 120 108; 4095 x 11776 263
+// 230 205.  At K 11776: 1023 x 2048 82.9 96.8 140; 2047 x 2048 139 121 150.
 int gemm_dense_thin(const GemmArgs& a, hipStream_t s) {
     auto tiles = [&](uint32_t rows) { return (a.s_rows + rows - 1u) / rows * static_cast<uint64_t>(a.n / 128u); };
     if (tiles(64u) <= 256u) {

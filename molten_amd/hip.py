@@ -593,8 +593,8 @@ def moe_route_batch(logits, bias, ids, gw, m: int, e: int, topk: int,
 class MoeTile:
     """Row x column tile of a grouped GEMM block map (src/kernels/quant.rs:19-40).
     T32 / T128 are the reference's shapes; GU128 / DN128 are MI355X tiles of
-    128 rows; GU512 / DN512 map whole expert segments of up to 512 rows (the
-    segment kernels the fused prefill uses for gate/up and down)."""
+    128 rows; GU512 / DN512 map expert segments of up to 512 rows (the fused
+    prefill's maps for gate/up and down)."""
 
     T32 = (32, 64)
     T128 = (128, 64)
@@ -696,7 +696,7 @@ def map_grid(n_entries: int, nt: int) -> int:
 def gemm_q4_grouped_ordered(a, w: QuantWeights, c, ord_map, n_entries: int, s_rows: int, n: int,
                             tile=MoeTile.DN512, stream=None) -> None:
     """The grouped GEMM over a launch-ordered block map (no reference
-    counterpart): entry b is workgroup b's; n_entries = map_grid(...)."""
+    counterpart): entries in launch order; n_entries = map_grid(...)."""
     check(load().mh_gemm_q4_grouped_ordered(_ptr(a), _qref(w), _ptr(c), _ptr(ord_map), n_entries, s_rows, n,
                                             tile[0], tile[1], _stream(stream)), "gemm_q4_grouped_ordered")
 

@@ -683,3 +683,27 @@ def test_dense_gemm_odd_groups(dev, orc, m, n, k):
     hip.gemm_q4_dense(to_dev(a), m, wd, c)
     blocks, nb = _dense_map(m, n)
     assert_close(from_dev(c, np.uint16), orc.gemm_q4_grouped(a, w, blocks, nb, n, 64), f"dense {m}x{n}x{k}")
+
+
+@pytest.mark.parametrize("m", [21, 700])
+def test_moe_prefill_unaligned_scales(dev, orc, m):
+    """Expert matrices whose scales and biases are 4 bytes past a 16-byte
+    boundary take the segment kernel on the launch-ordered maps: the bits of
+    the step with aligned ones."""
+    e, h, inter, topk = 16, 512, 512, 4
+    _log(f"moe prefill, scales 4 bytes off, m={m}")
+    rng = np.random.default_rng(m)
+    mats = moe_weights(rng, e, h, inter)
+    router = to_dev(router_weights(rng, e, h, f32=True))
+    bias = to_dev(rng.normal(0, 0.05, e).astype(np.float32))
+    x = to_dev(layout.synth_bf16(rng, (m, h)))
+    total, _ = hip.moe_prefill_workspace(m, e, topk, h, inter)
+    outs = []
+    for up in (dev_quant, lambda w: _dev_quant_off(w, 4)):
+        ws = [up(w) for w in mats]
+        work = zeros_dev((total // 4,), np.uint32)
+        out = zeros_dev((m, h), np.uint16)
+        hip.moe_prefill(router, bias, ws[0][0], ws[1][0], ws[2][0], e, topk, x, m, out, work, total, mode=0)
+        outs.append(from_dev(out, np.uint16))
+    assert outs[0].any()
+    np.testing.assert_array_equal(outs[0], outs[1])
