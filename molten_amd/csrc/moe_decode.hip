@@ -343,18 +343,21 @@ template <typename WT>
 int launch_router_tiles(const DenseArgs& a, hipStream_t stream) {
     // The smallest tile (tokens x experts) whose workgroups are few rounds of
     // the chip: a tile of 64 x 8 is a chain of ~17 us however few there are, a
-    // smaller one stages the experts' rows and x more often.  us by workgroups
-    // of the smaller tile, K 2048, 4 to 256 experts, f32 (bf16 the same):
-    // 16 x 2 against 16 x 8: 512 workgroups 5.4 / 7.5, 704 7.3 / 7.5, 800
-    // 8.6 / 7.6, 1024 8.6 / 7.7; 16 x 8 against 64 x 8: 800 15.7 / 19.4, 1024
-    // 16.0 / 18.1, 1280 20.9 / 20.4, 1408 22.3 / 20.8, 2048 29.5 / 21.6.
+    // smaller one stages the experts' rows and x more often, which costs less
+    // with short rows.  us by workgroups of the smaller tile, 4 to 256 experts,
+    // f32 (bf16 the same), K 2048: 16 x 2 against 16 x 8: 512 workgroups 5.4 /
+    // 7.5, 704 7.3 / 7.5, 800 8.6 / 7.6, 1024 8.6 / 7.7; 16 x 8 against 64 x 8:
+    // 800 15.7 / 19.4, 1024 16.0 / 18.1, 1280 20.9 / 20.4, 1408 22.3 / 20.8,
+    // 2048 29.5 / 21.6; K 1024: 1024 13.4 / 16.7, 1256 20.5 / 18.4, 1504 19.1 /
+    // 21.0, 1600 22.9 / 19.2.  K 512, 16 x 8 in parts of 64 x 8: 1024 0.75, 1256
+    // 0.87, 1536 0.87, 1600 1.10, 2048 1.17.
     auto tiles = [&](uint32_t tokens, uint32_t experts) {
         return static_cast<uint64_t>((a.m + tokens - 1u) / tokens) * ((a.n + experts - 1u) / experts);
     };
     if (tiles(16u, 2u) <= 768u) {
         return launch_router_tiles_as<WT, 16, 2>(a, stream);
     }
-    if (tiles(16u, 8u) <= 1024u) {
+    if (tiles(16u, 8u) <= (a.k <= 512u ? 1536u : 1024u)) {
         return launch_router_tiles_as<WT, 16, 8>(a, stream);
     }
     return launch_router_tiles_as<WT, 64, 8>(a, stream);

@@ -277,7 +277,7 @@ def test_prefill_router_and_route_batch(dev, orc):
     # tiles of 16 x 2 (odd experts, partial token tiles, the last count of
     # workgroups that takes them), of 16 x 8 from the next on, of 64 x 8
     (2, 3, 2048), (17, 17, 512), (512, 33, 1024), (12288, 2, 64), (12289, 2, 64), (700, 64, 2048), (801, 33, 1024),
-    (1025, 61, 2048), (2048, 64, 512), (2049, 64, 512), (1023, 131, 992), (16385, 3, 32)])
+    (1025, 61, 2048), (3072, 64, 512), (3073, 64, 512), (2049, 64, 544), (1023, 131, 992), (24577, 3, 32)])
 def test_prefill_router_tiles(dev, orc, m, e, k, f32):
     """Every tile of the prefill router gives the chunk-order logits, bit for bit."""
     _log(f"router {m}x{e}x{k} {'f32' if f32 else 'bf16'}")
