@@ -377,11 +377,12 @@ namespace mh {
 // there is one).  The segment kernel covers an expert of up to 288 rows in
 // one pass and dequantizes its codes once, but is level at best.  Steps with
 // 208 to 288 rows per expert in the mean, us on the segment kernel against
-// these: routed evenly, 64 experts of 2048 x 1536 368 to 424 / 378 to 424
-// (4096 tokens, by box and load: 4% faster to 3% slower), 128 experts 800 /
-// 780, 48 experts 306 / 271 (2.25 rounds of its workgroups); unevenly (a
-// selection bias), 64 experts 412 to 453 / 385 to 423, 128 experts 883 / 791,
-// 256 experts of 1024 x 512 519 / 468.  The host knows only the mean.
+// these: routed evenly, 64 experts of 2048 x 1536, 4096 tokens 368 to 393 / 378
+// to 390 in single passes (three boxes of four 2.5 to 4% slower here), 401 to
+// 412 / 388 to 389 with the clocks of a long run; 128 experts 802 / 792, 48
+// experts 331 / 302 (2.25 rounds of its workgroups); unevenly (a selection
+// bias), 64 experts 440 / 393, 128 experts 892 / 798, 256 experts of 1024 x 512
+// 519 / 468.  The host knows only the mean.
 bool thin_fits(const GemmArgs& a) {
     return a.ordered && a.stamps == nullptr && aligned(a.s0, 16) && aligned(a.b0, 16) && aligned(a.s1, 16) &&
            aligned(a.b1, 16);
