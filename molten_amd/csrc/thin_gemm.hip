@@ -378,7 +378,7 @@ namespace mh {
 // one pass and dequantizes its codes once, but is level at best.  Steps with
 // 208 to 288 rows per expert in the mean, us on the segment kernel against
 // these: routed evenly, 64 experts of 2048 x 1536, 4096 tokens 368 to 393 / 378
-// to 390 in single passes (three boxes of four 2.5 to 4% slower here), 401 to
+// to 390 in single passes (on three cards of four 2.5 to 4% slower here), 401 to
 // 412 / 388 to 389 with the clocks of a long run; 128 experts 802 / 792, 48
 // experts 331 / 302 (2.25 rounds of its workgroups); unevenly (a selection
 // bias), 64 experts 440 / 393, 128 experts 892 / 798, 256 experts of 1024 x 512
@@ -423,7 +423,7 @@ int gemm_grouped_thin(const GemmArgs& a, uint32_t n_entries, hipStream_t s) {
 
 // The dense product: the smallest tile that keeps one workgroup per CU, then
 // the widest (rows x columns of 64 x 128, 128 x 128, 128 x 256; us at K 2048,
-// one box, in a graph): 255 x 6144 15.7 20.2 27.2; 1023 x 2048 16.1 19.3 27.4;
+// one card, in a graph): 255 x 6144 15.7 20.2 27.2; 1023 x 2048 16.1 19.3 27.4;
 // 400 x 6144 23.3 21.1 29.0; 1023 x 6144 38.7 36.5 35.3; 2047 x 6144 71.6 61.4
 // 61.5; 4095 x 2048 50.3 42.3 40.9; 4095 x 6144 141 120 108; 4095 x 11776 263
 // 230 205.  At K 11776: 1023 x 2048 82.9 96.8 140; 2047 x 2048 139 121 150.
