@@ -375,7 +375,7 @@ namespace mh {
 // alignment limits checked as the segment kernel's): scales and biases are
 // read 16 bytes at a time (make_args leaves the second matrix's null where
 // there is one).  The segment kernel covers an expert of up to 288 rows in
-// one pass and dequantizes its codes once, but is level at best.  Steps with
+// one pass and dequantizes its codes once: a few percent at best.  Steps with
 // 208 to 288 rows per expert in the mean, us on the segment kernel against
 // these: routed evenly, 64 experts of 2048 x 1536, 4096 tokens 368 to 393 / 378
 // to 390 in single passes (on three cards of four 2.5 to 4% slower here), 401 to
